@@ -32,6 +32,42 @@ def test_dequant_bit_exact(E, K, N, linear):
             assert torch.equal(got[e].view(torch.uint8), want.contiguous().view(torch.uint8)), (e, dtype)
 
 
+# (E, K, N, G): one row past a tile of 32 packed rows and 8 columns past one of 64; the smallest;
+# the most groups the tile's table holds (64) and more; a group that a packed word straddles
+@pytest.mark.parametrize("E,K,N,G", [(2, 264, 72, 24), (3, 8, 8, 8), (1, 512, 136, 8),
+                                     (1, 1024, 64, 8), (2, 24, 16, 12)])
+@pytest.mark.parametrize("linear", [True, False])
+@pytest.mark.parametrize("act_order", [False, True])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_dequant_tile_edges(E, K, N, G, linear, act_order, offset):
+    """Bit-exact at the tile edges, with g_idx, and from bases that are not 16-byte aligned."""
+    _say(f"dequant tiles E={E} K={K} N={N} G={G} {linear} {act_order} {offset}")
+    g = torch.Generator().manual_seed(K + N)
+    q = torch.randint(-2**31, 2**31, (E, K // 8, N), generator=g).to(torch.int32)
+    z = torch.randint(-2**31, 2**31, (E, K // G, N // 8), generator=g).to(torch.int32)
+    s = (torch.randn(E, K // G, N, generator=g) * 0.05).half()
+    s[0, 0, :3] = torch.tensor([0.0, -6e-8, 65504.0]).half()
+    gi = torch.arange(K)[None].expand(E, K) // G
+    if act_order:
+        gi = gi[:, torch.randperm(K, generator=g)].contiguous()
+    nib = lambda t, d: torch.stack([(t >> (4 * j)) & 15 for j in range(8)], d + 1)  # noqa: E731
+    zero = nib(z, 2).reshape(E, K // G, N)
+    want = torch.stack([(nib(q[e], 0).reshape(K, N) - zero[e, gi[e]]).float() *
+                        s[e, gi[e]].float() for e in range(E)])
+    if linear:
+        want = want.transpose(1, 2).contiguous()
+
+    def dev(t):  # on the device, `offset` elements into its allocation
+        flat = torch.empty(t.numel() + offset, dtype=t.dtype, device="cuda")
+        flat[offset:] = t.reshape(-1).cuda()
+        return flat[offset:].view(t.shape)
+
+    for dtype in (torch.bfloat16, torch.float16, torch.float32):
+        got = ops.dequantize(dev(q), dev(z), dev(s), dev(gi.int()) if act_order else None,
+                             group_size=G, linear_weight=linear, dtype=dtype).cpu()
+        assert torch.equal(got, want.to(dtype)), dtype
+
+
 def test_dequant_reference_kat_and_g_idx():
     _say("dequant KAT")
     int_weight = (np.arange(16 * 8, dtype=np.int32).reshape(16, 8) % 16)
