@@ -62,6 +62,41 @@ def test_repack_is_bit_exact(layout, zeros, bf16):
         assert bool((got.qzeros == int(np.int32(np.uint32(0x88888888).view(np.int32)))).all())
 
 
+# (K, N, G): 5 packed rows and 9 columns past a 64-word tile; group counts that are and are not
+# multiples of 8; a whole tile and one word quad past it
+@pytest.mark.parametrize("K,N,G", [(40, 72, 8), (512, 64, 64), (544, 200, 32), (8, 8, 8)])
+@pytest.mark.parametrize("layout,bf16", [("wna16", False), ("wna16", True), ("awq", False)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_repack_tile_edges(K, N, G, layout, bf16, offset):
+    """The repack at the edges of its tiles, and from bases that are not 16-byte aligned."""
+    rng = np.random.default_rng(K + N)
+    E = 2
+    q, z, s = _rand_proj(rng, E, K, N, G)
+    if bf16:
+        s = torch.from_numpy(s).to(torch.bfloat16).float().numpy()
+
+    def dev(t):  # on the device, 4 bytes per `offset` into its allocation
+        skip = offset * 4 // t.element_size()
+        flat = torch.empty(t.numel() + skip, dtype=t.dtype, device="cuda")
+        flat[skip:] = t.reshape(-1).cuda()
+        return flat[skip:].view(t.shape)
+
+    if layout == "wna16":
+        b, zp, st = _wna16(q, z, s, bf16)
+        got = awq_to_gptq(dev(torch.from_numpy(b)), dev(torch.from_numpy(zp)), dev(st),
+                          layout=layout, in_features=K, group_size=G)
+    else:
+        qw = np.ascontiguousarray(np.stack([awq_ref.awq_pack_cols(q[e]) for e in range(E)]))
+        qz = np.ascontiguousarray(np.stack([awq_ref.awq_pack_cols(z[e]) for e in range(E)]))
+        got = awq_to_gptq(dev(torch.from_numpy(qw)), dev(torch.from_numpy(qz)),
+                          dev(torch.from_numpy(s.astype(np.float16))), layout=layout,
+                          in_features=K, group_size=G)
+    for e in range(E):
+        assert np.array_equal(got.qweight[e].cpu().numpy(), gptq_ref.pack_rows(q[e].astype(np.int32)))
+        assert np.array_equal(got.qzeros[e].cpu().numpy(), gptq_ref.pack_cols(z[e].astype(np.int32)))
+        assert np.array_equal(got.scales[e].float().cpu().numpy(), s[e])
+
+
 def test_layer_on_awq_experts_matches_the_oracle():
     """16 AWQ (wna16) experts repacked on the GPU run through the routed layer; the oracle layer
     is computed from the oracle's own repack of the same AWQ tensors."""
