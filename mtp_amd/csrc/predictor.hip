@@ -4,17 +4,69 @@
 // The reference's predictor (src/mtp_expert_prefetch/training/hidden_residual.py:44-106,
 // Linear -> SiLU -> ... -> Linear(w, E), one prediction per layer) is simplified, as the offload
 // workload specifies, to a two-layer bf16 MLP per layer with random weights whose top-16 experts
-// drive the prefetch of that layer. All heads run in four launches: the first products of every
-// head as one [T, L*D] GEMV (w1 heads are contiguous rows), SiLU into a head-major activation,
-// the second products with the head on grid.y, and one wave per (head, token) for the top-k.
-// Both products use the canonical fp32 dot order of the router (routing.h:logits_tile); the
-// hidden activation is SiLU in fp32 rounded once to bf16 (the bf16 Linear output dtype).
+// drive the prefetch of that layer. All heads run in three launches: the first products of every
+// head as one [T, L*D] product (w1 heads are contiguous rows) with SiLU into a head-major
+// activation, the second products with the head on grid.y, and one wave per (head, token) for the
+// top-k. Both products use the canonical fp32 dot order of the router (routing.h:logits_tile);
+// the hidden activation is SiLU in fp32 rounded once to bf16 (the bf16 Linear output dtype).
 #include "launch.h"
 #include "routing.h"
 
 namespace {
 
-// out[head][t][n] (row stride N + 1) = x[head][t][:] . W[head][n][:], head = blockIdx.y.
+// bf16(silu(v)).
+MOE_DEV uint16_t silu_bf16(float v) { return (uint16_t)f32_to_bf16_rne(v / (1.0f + expf(-v))); }
+
+// x[head][t][:] . W[head][n][:] for the 4 waves x TE rows n of a workgroup, head = blockIdx.y, and
+// the token tiles of its kTokensPerWg tokens: every wave issues the loads of its
+// weight rows, then each tile of TT token rows passes through LDS, so a weight row is read once for
+// kTokensPerWg tokens and the whole 16 KB of a wave's rows is in flight at once (bound by HBM up to
+// about 8 tokens, by the fp32 FMAs beyond). Reading the row from memory once per token took 95 us
+// for the first product of 40 heads (168 MB) at 4 tokens.
+// ACT: out is bf16 [n / D][T][D] = silu(z); else fp32 [head][T][N + 1].
+constexpr int kRowsTE = 4, kTokensPerWg = 32;
+template <int TT, int NI, bool ACT>
+__global__ __launch_bounds__(256) void mlp_rows_kernel(const uint16_t* __restrict__ x,
+                                                       int64_t x_head, int T, int K,
+                                                       const uint16_t* __restrict__ W,
+                                                       int64_t w_head, int N, int D,
+                                                       void* __restrict__ out_v) {
+  __shared__ __attribute__((aligned(16))) uint16_t s_x[TT * NI * 512];
+  constexpr int NV = TT * kRowsTE;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t head = blockIdx.y;
+  const int row_blocks = (N + 4 * kRowsTE - 1) / (4 * kRowsTE);
+  const int n0 = ((int)blockIdx.x % row_blocks * 4 + wave) * kRowsTE;
+  LdsLogitsTile<TT, kRowsTE, NI> tile;
+  tile.load(K, W + head * w_head, N, nullptr, n0, lane);
+  const __amdgpu_buffer_rsrc_t xr = buf_rsrc(x + head * x_head, (uint32_t)T * (uint32_t)K * 2u);
+  const int t_begin = (int)blockIdx.x / row_blocks * kTokensPerWg;
+  const int t_end = min(T, t_begin + kTokensPerWg);
+  for (int t0 = t_begin; t0 < t_end; t0 += TT) {
+    if (t0 > t_begin) __syncthreads();  // the previous tile is read
+    // the tile's rows are contiguous; past the last token the loads read zeros
+#pragma unroll
+    for (int u = 0; u < (TT * NI + 3) / 4; ++u) {
+      const int o = 8 * (tid + 256 * u);
+      if (o < TT * K)
+        *reinterpret_cast<u32x4*>(s_x + o) = buf_ld128(xr, ((uint32_t)t0 * K + o) * 2u);
+    }
+    __syncthreads();
+    float acc[NV];
+    tile.partials(s_x, K, lane, acc);
+    fold_partials(acc, lane);
+    const int v = lane / (64 / NV), t = t0 + v / kRowsTE, n = n0 + v % kRowsTE;
+    if (lane % (64 / NV) == 0 && t < t_end && n < N) {
+      if constexpr (ACT)
+        static_cast<uint16_t*>(out_v)[((int64_t)(n / D) * T + t) * D + n % D] = silu_bf16(acc[0]);
+      else
+        static_cast<float*>(out_v)[(head * T + t) * (N + 1) + n] = acc[0];
+    }
+  }
+}
+
+// The same products for any K: one wave per TT x TE tile, out[head][t][n] fp32 (row stride N + 1).
 template <int TT, int TE>
 __global__ __launch_bounds__(256) void mlp_logits_kernel(
     const uint16_t* __restrict__ x, int64_t x_head, int T, int K, const uint16_t* __restrict__ W,
@@ -38,8 +90,7 @@ __global__ void silu_bf16_kernel(const float* __restrict__ z, int T, int L, int 
   if (i >= per_head * L) return;
   const int64_t l = i / per_head, r = i % per_head;
   const int64_t t = r / D, j = r % D;
-  const float v = z[t * ((int64_t)L * D + 1) + l * D + j];
-  a[i] = (uint16_t)f32_to_bf16_rne(v / (1.0f + expf(-v)));
+  a[i] = silu_bf16(z[t * ((int64_t)L * D + 1) + l * D + j]);
 }
 
 // One wave per (head, token): logits row (head * T + t) of z2, ids/scores [head][t][top_k].
@@ -66,20 +117,52 @@ hipError_t launch_mlp_logits(const uint16_t* x, int64_t x_head, int T, int K, co
   return hipGetLastError();
 }
 
+// The tiled products hold K in at most four 512-column steps per lane.
+constexpr int kRowsMaxK = 2048;
+
+template <int NI, bool ACT>
+hipError_t launch_mlp_rows(const uint16_t* x, int64_t x_head, int T, int K, const uint16_t* W,
+                           int64_t w_head, int N, int D, void* out, int heads,
+                           hipStream_t stream) {
+  const unsigned row_blocks = (N + 4 * kRowsTE - 1) / (4 * kRowsTE);
+  const dim3 grid(row_blocks * ((T + kTokensPerWg - 1) / kTokensPerWg), heads);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, x_head, T, K, W, w_head, N, D, out);
+    return hipGetLastError();
+  };
+  // the token tile nearest to the batch: rows of a larger one would be zeros
+  if (T == 1) return go(mlp_rows_kernel<1, NI, ACT>);
+  if (T == 2) return go(mlp_rows_kernel<2, NI, ACT>);
+  if (T <= 4) return go(mlp_rows_kernel<4, NI, ACT>);
+  return go(mlp_rows_kernel<8, NI, ACT>);
+}
+
 }  // namespace
 
 hipError_t launch_predictor(const uint16_t* h, int T, int H, int L, const uint16_t* w1, int D,
                             const uint16_t* w2, int E, int top_k, float* z1, uint16_t* a,
                             float* z2, int32_t* ids, float* scores, hipStream_t stream) {
   const int LD = L * D;
-  hipError_t err = launch_mlp_logits<1, 2>(h, 0, T, H, w1, 0, LD, z1, 0, 1, stream);
+  hipError_t err;
+  if (H <= kRowsMaxK) {
+    err = H <= 1024 ? launch_mlp_rows<2, true>(h, 0, T, H, w1, 0, LD, D, a, 1, stream)
+                    : launch_mlp_rows<4, true>(h, 0, T, H, w1, 0, LD, D, a, 1, stream);
+  } else {
+    err = launch_mlp_logits<1, 2>(h, 0, T, H, w1, 0, LD, z1, 0, 1, stream);
+    if (err != hipSuccess) return err;
+    const int64_t n = (int64_t)T * LD;
+    hipLaunchKernelGGL(silu_bf16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
+                       z1, T, L, D, a);
+    err = hipGetLastError();
+  }
   if (err != hipSuccess) return err;
-  const int64_t n = (int64_t)T * LD;
-  hipLaunchKernelGGL(silu_bf16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, z1,
-                     T, L, D, a);
-  if ((err = hipGetLastError()) != hipSuccess) return err;
-  err = launch_mlp_logits<1, 2>(a, (int64_t)T * D, T, D, w2, (int64_t)E * D, E, z2,
-                                (int64_t)T * (E + 1), L, stream);
+  const int64_t x2 = (int64_t)T * D, w2h = (int64_t)E * D;
+  if (D <= 1024)
+    err = launch_mlp_rows<2, false>(a, x2, T, D, w2, w2h, E, D, z2, L, stream);
+  else if (D <= kRowsMaxK)
+    err = launch_mlp_rows<4, false>(a, x2, T, D, w2, w2h, E, D, z2, L, stream);
+  else
+    err = launch_mlp_logits<1, 2>(a, x2, T, D, w2, w2h, E, z2, (int64_t)T * (E + 1), L, stream);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL(predictor_topk_kernel, dim3((T * L + 3) / 4), dim3(256), 0, stream, z2, T, L,
                      E, top_k, ids, scores);

@@ -100,55 +100,9 @@ hipError_t launch_logits_norm(const uint16_t* res_in, const uint16_t* add, const
 // loads of step s + 1 are issued before the arithmetic of step s, and the kernel keeps at most
 // 256 VGPRs so two waves share each SIMD.
 //
-// The 64 per-lane partials are then combined by a transposed butterfly: at the step of lane
-// mask m every lane keeps the half of its values whose index bit matches its own lane bit and
-// adds the partner's (lane ^ m) copy of the same values. Every addition is the one the
-// butterfly v += shfl_xor(v, m) makes at that lane (the same two operands, and fp32 addition is
-// commutative), so the result is bit-identical, with 63 exchanges instead of 6 x 64. After the
-// last step lane l holds value l = (token i = l >> 3, row j = l & 7).
+// The 64 per-lane partials are then combined by a transposed butterfly (fold_partials), after
+// which lane l holds value l = (token i = l >> 3, row j = l & 7).
 constexpr int kRowsTileT = 8, kRowsTileE = 8;
-
-template <int N, int HALF>
-MOE_DEV void fold_swap32(float (&a)[N]) {
-#pragma unroll
-  for (int v = 0; v < HALF; ++v) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[v]),
-                                                    __float_as_uint(a[v + HALF]), false, false);
-    a[v] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-}
-
-template <int N, int HALF>
-MOE_DEV void fold_swap16(float (&a)[N]) {
-#pragma unroll
-  for (int v = 0; v < HALF; ++v) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[v]),
-                                                    __float_as_uint(a[v + HALF]), false, false);
-    a[v] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
-}
-
-// Lane mask M in {8, 4, 2, 1}: rows of 16 lanes, exchanged with DPP.
-template <int M, int N>
-MOE_DEV void fold_dpp(float (&a)[N], int lane) {
-  const bool up = (lane & M) != 0;
-#pragma unroll
-  for (int v = 0; v < M; ++v) {
-    const float keep = up ? a[v + M] : a[v];
-    const int send = __float_as_int(up ? a[v] : a[v + M]);
-    int recv;
-    if constexpr (M == 8) {
-      recv = __builtin_amdgcn_update_dpp(0, send, 0x128, 0xF, 0xF, false);  // row_ror:8
-    } else if constexpr (M == 4) {
-      recv = __shfl_xor(send, 4, 64);  // no single row DPP pattern pairs lane i with i ^ 4
-    } else if constexpr (M == 2) {
-      recv = __builtin_amdgcn_update_dpp(0, send, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
-    } else {
-      recv = __builtin_amdgcn_update_dpp(0, send, 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
-    }
-    a[v] = keep + __int_as_float(recv);
-  }
-}
 
 MOE_DEV float bf16_elem(const u32x4& v, int el) {
   return (el & 1) ? bf16hi_to_f32(v[el >> 1]) : bf16lo_to_f32(v[el >> 1]);
@@ -225,12 +179,7 @@ __global__ __launch_bounds__(256, 2) void router_logits_rows_kernel(
   }
   if (nsteps & 1) compute(xa, wa);
 
-  fold_swap32<TT * TE, 32>(acc);
-  fold_swap16<TT * TE, 16>(acc);
-  fold_dpp<8>(acc, lane);
-  fold_dpp<4>(acc, lane);
-  fold_dpp<2>(acc, lane);
-  fold_dpp<1>(acc, lane);
+  fold_partials(acc, lane);
 
   const int t = t0 + (lane >> 3), e = e0 + (lane & 7);
   if (t < T && e < rows) {

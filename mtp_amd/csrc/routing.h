@@ -16,6 +16,46 @@
 #include "common.h"
 
 // ---------------------------------------------------------------------------- logits
+// NV <= 64 (a power of two) values of partial sums per lane, summed over the lanes by a
+// transposed butterfly: at the step of lane mask m every lane keeps the half of its values whose
+// index bit matches its own lane bit and adds the partner's (lane ^ m) copy of the same values;
+// once one value is left, the remaining masks are plain butterfly steps. Every addition is the
+// one the butterfly v += shfl_xor(v, m) makes at that lane (the same two operands, and fp32
+// addition is commutative), so the sums are bit-identical to it, with NV - 1 exchanges plus the
+// plain steps instead of 6 NV. Afterwards a[0] of lane l is the sum of value l / (64 / NV).
+template <int M, int HALF, int N>
+MOE_DEV void fold_step(float (&a)[N], int lane) {
+  if constexpr (HALF == 0) {
+    a[0] = a[0] + xor_partner<M>(a[0]);
+  } else {
+    const bool up = (lane & M) != 0;
+#pragma unroll
+    for (int v = 0; v < HALF; ++v) {
+      if constexpr (M == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[v]),
+                                                        __float_as_uint(a[v + HALF]), false, false);
+        a[v] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      } else if constexpr (M == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[v]),
+                                                        __float_as_uint(a[v + HALF]), false, false);
+        a[v] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      } else {
+        const float keep = up ? a[v + HALF] : a[v];
+        a[v] = keep + xor_partner<M>(up ? a[v] : a[v + HALF]);
+      }
+    }
+  }
+}
+template <int NV>
+MOE_DEV void fold_partials(float (&a)[NV], int lane) {
+  fold_step<32, NV / 2>(a, lane);
+  fold_step<16, NV / 4>(a, lane);
+  fold_step<8, NV / 8>(a, lane);
+  fold_step<4, NV / 16>(a, lane);
+  fold_step<2, NV / 32>(a, lane);
+  fold_step<1, NV / 64>(a, lane);
+}
+
 template <int TT, int TE>
 MOE_DEV void logits_tile(const uint16_t* __restrict__ x, int T, int H, const uint16_t* __restrict__ W,
                          int E, const uint16_t* __restrict__ shared_w, const float* __restrict__ bias,
@@ -104,9 +144,9 @@ MOE_DEV void logits_tile(const uint16_t* __restrict__ x, int T, int H, const uin
 // t0 + TT - 1 of the batch), in two phases: load() issues every chunk of the wave's TE router
 // rows (no dependence on x), compute_store() runs the same chunks per lane, fma order and
 // butterfly as logits_tile, so the logits are bit-identical to logits_tile on the same rows.
-template <int TT, int TE>
+template <int TT, int TE, int NI_ = 4>
 struct LdsLogitsTile {
-  static constexpr int NI = 4;  // 64 * NI chunks of 8 = 2048 columns
+  static constexpr int NI = NI_;  // 64 * NI chunks of 8 columns
   u32x4 wv[NI][TE];
 
   MOE_DEV void load(int H, const uint16_t* __restrict__ W, int E,
@@ -128,15 +168,11 @@ struct LdsLogitsTile {
     }
   }
 
-  MOE_DEV void compute_store(const uint16_t* x_lds, int T, int H, int E, bool has_shared,
-                             const float* __restrict__ bias, float* __restrict__ logits, int t0,
-                             int e0, int lane) const {
-    const int rows = E + (has_shared ? 1 : 0), nq = H / 8;
-    float acc[TT][TE];
+  // acc[i * TE + j]: the lane's partial of (token i, row j) over its chunks.
+  MOE_DEV void partials(const uint16_t* x_lds, int H, int lane, float (&acc)[TT * TE]) const {
+    const int nq = H / 8;
 #pragma unroll
-    for (int i = 0; i < TT; ++i)
-#pragma unroll
-      for (int j = 0; j < TE; ++j) acc[i][j] = 0.0f;
+    for (int v = 0; v < TT * TE; ++v) acc[v] = 0.0f;
 #pragma unroll
     for (int it = 0; it < NI; ++it) {
       const int q = 64 * it + lane;
@@ -155,18 +191,21 @@ struct LdsLogitsTile {
           const uint32_t xd = xv[i][el >> 1];
           const float xf = (el & 1) ? bf16hi_to_f32(xd) : bf16lo_to_f32(xd);
 #pragma unroll
-          for (int j = 0; j < TE; ++j) acc[i][j] = __builtin_fmaf(xf, wf[j], acc[i][j]);
+          for (int j = 0; j < TE; ++j)
+            acc[i * TE + j] = __builtin_fmaf(xf, wf[j], acc[i * TE + j]);
         }
       }
     }
+  }
+
+  MOE_DEV void compute_store(const uint16_t* x_lds, int T, int H, int E, bool has_shared,
+                             const float* __restrict__ bias, float* __restrict__ logits, int t0,
+                             int e0, int lane) const {
+    const int rows = E + (has_shared ? 1 : 0);
+    float acc[TT * TE];
+    partials(x_lds, H, lane, acc);
 #pragma unroll
-    for (int i = 0; i < TT; ++i)
-#pragma unroll
-      for (int j = 0; j < TE; ++j) {
-        float v = acc[i][j];
-        v = bfly_sum(v);
-        acc[i][j] = v;
-      }
+    for (int v = 0; v < TT * TE; ++v) acc[v] = bfly_sum(acc[v]);
     if (lane == 0) {
 #pragma unroll
       for (int i = 0; i < TT; ++i)
@@ -174,7 +213,7 @@ struct LdsLogitsTile {
         for (int j = 0; j < TE; ++j) {
           const int t = t0 + i, e = e0 + j;
           if (t < T && e < rows) {
-            float v = acc[i][j];
+            float v = acc[i * TE + j];
             if (bias && e < E) v = v + bias[e];
             logits[(int64_t)t * (E + 1) + e] = v;
           }

@@ -181,6 +181,28 @@ def test_predictor_matches_oracle(T, L, H, D, E, k):
                     assert abs(la - lb) <= 1e-4 * max(abs(lb), 1e-3), (l, t, j, a, b, la, lb)
 
 
+# widths at, below and past the 512-column steps, one past the widest tiled row (2048 -> 2056)
+@pytest.mark.parametrize("H,D", [(64, 32), (520, 1032), (1024, 512), (2048, 2048), (2056, 2056)])
+def test_predictor_batches_equal_single_tokens(H, D):
+    """The logits keep the canonical summation order whatever the token tile: every token's ids in
+    a batch (one that ends inside a tile and in a second workgroup's tokens) are those of the
+    token alone, and the oracle's up to near-ties."""
+    L, E, k, T = 3, 40, 8, 37
+    g = torch.Generator().manual_seed(H)
+    h = torch.randn(T, H, generator=g).to(torch.bfloat16)
+    w1 = (torch.randn(L, D, H, generator=g) * 0.02).to(torch.bfloat16)
+    w2 = (torch.randn(L, E, D, generator=g) * 0.02).to(torch.bfloat16)
+    dev = [t.cuda() for t in (h, w1, w2)]
+    single = torch.cat([ops.predictor_topk(dev[0][t:t + 1], *dev[1:], k) for t in range(T)], dim=1)
+    for n in (2, 3, 5, 8, 9, 32, T):
+        _say(f"predictor H={H} D={D} batch {n}")
+        assert torch.equal(ops.predictor_topk(dev[0][:n].contiguous(), *dev[1:], k), single[:, :n]), n
+    r_ids, r_logits = moe_ref.predictor_ref(bf16_bits(h[:2]), bf16_bits(w1), bf16_bits(w2), k)
+    for l, t, j in np.argwhere(single[:, :2].cpu().numpy() != r_ids):
+        la, lb = r_logits[l, t, int(single[l, t, j])], r_logits[l, t, r_ids[l, t, j]]
+        assert abs(la - lb) <= 1e-4 * max(abs(lb), 1e-3), (l, t, j)
+
+
 def test_predictor_rejects_bad_shapes():
     h = torch.zeros(1, 64, dtype=torch.bfloat16, device="cuda")
     w1 = torch.zeros(2, 32, 64, dtype=torch.bfloat16, device="cuda")
