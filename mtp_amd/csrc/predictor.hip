@@ -19,12 +19,14 @@ MOE_DEV uint16_t silu_bf16(float v) { return (uint16_t)f32_to_bf16_rne(v / (1.0f
 
 // x[head][t][:] . W[head][n][:] for the 4 waves x TE rows n of a workgroup, head = blockIdx.y, and
 // the token tiles of its kTokensPerWg tokens: every wave issues the loads of its
-// weight rows, then each tile of TT token rows passes through LDS, so a weight row is read once for
-// kTokensPerWg tokens and the whole 16 KB of a wave's rows is in flight at once (bound by HBM up to
-// about 8 tokens, by the fp32 FMAs beyond). Reading the row from memory once per token took 95 us
-// for the first product of 40 heads (168 MB) at 4 tokens.
+// weight rows, then each tile of TT token rows passes through LDS, so a weight row is read once
+// for kTokensPerWg tokens and the whole 8 KB of a wave's rows is in flight at once (bound by HBM up
+// to about 4 tokens, by the fp32 FMAs beyond). 40 heads (2048 -> 1024 -> 256, 189 MB) per call:
+// 4 tokens 116.7 -> 50.6 us (the row read from memory once per token before), 1 token 37.5 us, 16
+// tokens 89 us. Two rows per wave (four: 58.3 us at 4 tokens, one: 57.4) and nontemporal
+// weight loads (53.5 -> 50.6).
 // ACT: out is bf16 [n / D][T][D] = silu(z); else fp32 [head][T][N + 1].
-constexpr int kRowsTE = 4, kTokensPerWg = 32;
+constexpr int kRowsTE = 2, kTokensPerWg = 32;
 template <int TT, int NI, bool ACT>
 __global__ __launch_bounds__(256) void mlp_rows_kernel(const uint16_t* __restrict__ x,
                                                        int64_t x_head, int T, int K,
@@ -38,7 +40,7 @@ __global__ __launch_bounds__(256) void mlp_rows_kernel(const uint16_t* __restric
   const int64_t head = blockIdx.y;
   const int row_blocks = (N + 4 * kRowsTE - 1) / (4 * kRowsTE);
   const int n0 = ((int)blockIdx.x % row_blocks * 4 + wave) * kRowsTE;
-  LdsLogitsTile<TT, kRowsTE, NI> tile;
+  LdsLogitsTile<TT, kRowsTE, NI, kBufNontemporal> tile;
   tile.load(K, W + head * w_head, N, nullptr, n0, lane);
   const __amdgpu_buffer_rsrc_t xr = buf_rsrc(x + head * x_head, (uint32_t)T * (uint32_t)K * 2u);
   const int t_begin = (int)blockIdx.x / row_blocks * kTokensPerWg;
@@ -130,11 +132,11 @@ hipError_t launch_mlp_rows(const uint16_t* x, int64_t x_head, int T, int K, cons
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, x_head, T, K, W, w_head, N, D, out);
     return hipGetLastError();
   };
-  // the token tile nearest to the batch: rows of a larger one would be zeros
+  // the token tile nearest to the batch: rows of a larger one would be zeros. 4 tokens at most:
+  // tiles of 8 cost registers (8 tokens 68.2 vs 61.7 us a call, 16 tokens 98.1 vs 88.7)
   if (T == 1) return go(mlp_rows_kernel<1, NI, ACT>);
   if (T == 2) return go(mlp_rows_kernel<2, NI, ACT>);
-  if (T <= 4) return go(mlp_rows_kernel<4, NI, ACT>);
-  return go(mlp_rows_kernel<8, NI, ACT>);
+  return go(mlp_rows_kernel<4, NI, ACT>);
 }
 
 }  // namespace

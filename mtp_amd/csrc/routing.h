@@ -144,7 +144,8 @@ MOE_DEV void logits_tile(const uint16_t* __restrict__ x, int T, int H, const uin
 // t0 + TT - 1 of the batch), in two phases: load() issues every chunk of the wave's TE router
 // rows (no dependence on x), compute_store() runs the same chunks per lane, fma order and
 // butterfly as logits_tile, so the logits are bit-identical to logits_tile on the same rows.
-template <int TT, int TE, int NI_ = 4>
+// AUX: cache policy of the weight loads.
+template <int TT, int TE, int NI_ = 4, int AUX = 0>
 struct LdsLogitsTile {
   static constexpr int NI = NI_;  // 64 * NI chunks of 8 columns
   u32x4 wv[NI][TE];
@@ -163,7 +164,7 @@ struct LdsLogitsTile {
       for (int it = 0; it < NI; ++it) {
         const int q = 64 * it + lane;
         const uint32_t qo = q < nq ? (uint32_t)q * 16u : kOutOfRange;
-        wv[it][j] = buf_ld128(e == E ? sr : wr, (wo + qo) | (qo & kOutOfRange));
+        wv[it][j] = buf_ld128<AUX>(e == E ? sr : wr, (wo + qo) | (qo & kOutOfRange));
       }
     }
   }
