@@ -414,6 +414,29 @@ def test_hidden_residual_predictor_matches_oracle(scope):
         m(h.cuda(), layer_ids=lid[:2])
 
 
+# (N, H, W, F, E): one row; a row past 16 with 3 rows per example; widths and experts that end
+# inside a 32-k step, a 64-lane column and a 16-expert tile; the widest context, 512 experts
+@pytest.mark.parametrize("N,H,W,F,E,k", [(1, 64, 64, 1, 4, 2), (17, 520, 264, 3, 260, 16),
+                                         (11, 2048, 72, 3, 40, 8), (6, 1024, 1024, 7, 512, 64),
+                                         (40, 2056, 256, 1, 100, 1)])
+def test_hidden_residual_predictor_tile_edges(N, H, W, F, E, k):
+    from mtp_amd.predictor import HiddenResidualExpertPredictor
+    _say(f"hidden-residual predictor N={N} H={H} W={W} F={F} E={E} k={k}")
+    m = HiddenResidualExpertPredictor(hidden_size=H, num_experts=E, num_layers=5, future_window=F,
+                                      width=W, seed=N)
+    g = torch.Generator().manual_seed(W)
+    h = torch.randn(N, H, generator=g).to(torch.bfloat16)
+    lid = (torch.arange(N) % 5).to(torch.int32)
+    prior = torch.randn(N, F, E, generator=g)
+    ids, out = m.predict_topk(h.cuda(), layer_ids=lid, k=k, prior=prior, return_logits=True)
+    r_ids, r_out, _ = moe_ref.hidden_residual_ref(bf16_bits(h), _hr_oracle_params(m), lid.numpy(),
+                                                  top_k=k, prior=prior.numpy())
+    # a bf16 activation that rounds the other way (2^-8 of |g| <= 4, times a weight of the
+    # classifier's scale) moves a logit; the default shape's tolerance
+    assert np.max(np.abs(out.cpu().numpy() - r_out)) <= 1e-2
+    _ids_match_up_to_near_ties(ids.cpu().numpy(), r_ids, r_out, 2e-2)
+
+
 def test_hidden_residual_predictor_loads_a_reference_state_dict():
     """Parameters in the reference module's state_dict names: the forward then agrees with the
     same architecture built from torch's layers in fp32 (to bf16 accuracy)."""
