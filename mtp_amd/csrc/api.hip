@@ -161,15 +161,15 @@ enum Routing {
   ROUTE_GRID_IDS        // slot grid over the ids/weights in place
 };
 
-// [align ->] W1 -> W2 -> top-k sum over a routed workspace.
+// [align ->] W1 -> W2 -> top-k sum over a workspace. ids [T * top_k] and w [T * top_k (+ T shared
+// gates)] are the routing: the workspace's own, or a caller's arrays (read only: every form but
+// ROUTE_GRID_LOGITS, which publishes its top-k to them).
 int run_experts(const uint16_t* x, int T, int top_k, const moe_expert_set_v1* ex,
-                const moe_expert_set_v1* sh, const Workspace& L, void* ws, uint16_t* out,
-                int path, Routing routing, hipStream_t stream) {
+                const moe_expert_set_v1* sh, const Workspace& L, void* ws, int32_t* ids, float* w,
+                uint16_t* out, int path, Routing routing, hipStream_t stream) {
   const int has_shared = sh ? 1 : 0;
   const ExpertsDev ed = make_experts_dev(ex, sh);
   SlotsDev sd{T, top_k, T * top_k + (has_shared ? T : 0)};
-  int32_t* ids = at<int32_t>(ws, L.ids);
-  float* w = at<float>(ws, L.w);
   int32_t* sorted = at<int32_t>(ws, L.sorted);
   int32_t* eids = at<int32_t>(ws, L.eids);
   int32_t* ntpp = at<int32_t>(ws, L.ntpp);
@@ -531,7 +531,7 @@ int layer_impl(const uint16_t* x, int32_t T, const uint16_t* router_w, const flo
                                         shared ? shared_gate_w : nullptr, logit_bias, top_k,
                                         logits, at<float>(workspace, L.norms), ids, w, s),
                   "router (prefill)");
-    rc = run_experts(x, T, top_k, experts, shared, L, workspace, out, path, ROUTE_ALIGN, s);
+    rc = run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, out, path, ROUTE_ALIGN, s);
     if (rc) return rc;
     return copy_routing(ids, w, T, top_k, topk_ids_out, topk_weights_out, s);
   }
@@ -565,7 +565,7 @@ int layer_impl(const uint16_t* x, int32_t T, const uint16_t* router_w, const flo
     MOE_CHECK_HIP(launch_router_topk(logits, T, E, top_k, shared ? 1 : 0, ids, w, s),
                   "router topk");
   }
-  rc = run_experts(x, T, top_k, experts, shared, L, workspace, out, path, routing, s);
+  rc = run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, out, path, routing, s);
   if (rc) return rc;
   return copy_routing(ids, w, T, top_k, topk_ids_out, topk_weights_out, s);
 }
@@ -641,19 +641,38 @@ int moe_fused_experts_v1(const uint16_t* x, int32_t T, const int32_t* topk_ids,
   if (!workspace_aligned(workspace))
     return fail(MOE_ERR_WORKSPACE, "experts: workspace must be 256-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  int32_t* ids = at<int32_t>(workspace, L.ids);
-  float* w = at<float>(workspace, L.w);
-  MOE_CHECK_HIP(hipMemcpyAsync(ids, topk_ids, (size_t)T * top_k * 4, hipMemcpyDeviceToDevice, s),
-                "copy ids");
-  MOE_CHECK_HIP(hipMemcpyAsync(w, topk_weights, (size_t)T * top_k * 4, hipMemcpyDeviceToDevice, s),
-                "copy weights");
-  if (shared)
+  // The kernels read the caller's routing in place (copied to the workspace first it cost two
+  // launches: eight routed layers of 48 tokens, hidden 1024, 197 -> 169 us). With a shared
+  // expert its gate kernel writes the gates behind the routed weights, so those move to the
+  // workspace in that launch. A routing that shares bytes with the output, which the last kernels
+  // write while others still read the routing, is copied as a whole.
+  const size_t n = (size_t)T * top_k;
+  auto in_out = [&](const void* p, size_t bytes) {
+    const uintptr_t a = (uintptr_t)p, o = (uintptr_t)out;
+    return a < o + (size_t)T * experts->hidden * 2 && o < a + bytes;
+  };
+  const bool copy = in_out(topk_ids, n * 4) || in_out(topk_weights, n * 4);
+  int32_t* ids = const_cast<int32_t*>(topk_ids);
+  float* w = const_cast<float*>(topk_weights);
+  if (copy) {
+    ids = at<int32_t>(workspace, L.ids);
+    w = at<float>(workspace, L.w);
+    MOE_CHECK_HIP(hipMemcpyAsync(ids, topk_ids, n * 4, hipMemcpyDeviceToDevice, s), "copy ids");
+    MOE_CHECK_HIP(hipMemcpyAsync(w, topk_weights, n * 4, hipMemcpyDeviceToDevice, s),
+                  "copy weights");
+  }
+  if (shared) {
+    float* wsh = at<float>(workspace, L.w);
     MOE_CHECK_HIP(launch_shared_gate(x, T, experts->hidden, shared_gate_w, top_k,
-                                     at<float>(workspace, L.logits), w, s), "shared gate");
+                                     at<float>(workspace, L.logits), copy ? nullptr : topk_weights,
+                                     wsh, s),
+                  "shared gate");
+    w = wsh;
+  }
   const Routing routing = (path == MOE_PATH_DECODE && slot_grid_fits(T, top_k, shared ? 1 : 0))
                               ? ROUTE_GRID_IDS
                               : ROUTE_ALIGN;
-  return run_experts(x, T, top_k, experts, shared, L, workspace, out, path, routing, s);
+  return run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, out, path, routing, s);
 }
 
 }  // extern "C"
@@ -753,7 +772,7 @@ int moe_offload_layer_v1(uint64_t cache, int32_t layer, const uint16_t* x, int32
   if (rc) return rc;
   const Routing routing =
       (path == MOE_PATH_DECODE && slot_grid_fits(T, top_k, 0)) ? ROUTE_GRID_IDS : ROUTE_ALIGN;
-  rc = run_experts(x, T, top_k, experts, nullptr, L, workspace, out, path, routing, s);
+  rc = run_experts(x, T, top_k, experts, nullptr, L, workspace, ids, w, out, path, routing, s);
   if (rc) return rc;
   // The wait for the ids drained the compute stream, and the demand's slots (the only ones the
   // kernels just enqueued read) stay pinned until layer_done: the prefetch needs no ordering

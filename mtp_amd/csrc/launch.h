@@ -70,7 +70,8 @@ hipError_t launch_topk_align(const float* logits, int T, int E, int top_k, int h
                              int cap, int32_t* ids, float* weights, int32_t* sorted, int32_t* eids,
                              int32_t* ntpp, hipStream_t stream);
 hipError_t launch_shared_gate(const uint16_t* x, int T, int H, const uint16_t* shared_w,
-                              int top_k, float* logits_ws, float* weights, hipStream_t stream);
+                              int top_k, float* logits_ws, const float* routed, float* weights,
+                              hipStream_t stream);
 
 int align_capacity_blocks(int T, int top_k, int E, int has_shared, int BM);
 // Bytes of scratch (outside the output buffers) that lets launch_align spread the large-input

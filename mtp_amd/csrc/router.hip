@@ -295,24 +295,28 @@ hipError_t launch_topk_align(const float* logits, int T, int E, int top_k, int h
   return hipGetLastError();
 }
 
-// Shared-gate only (no routed experts): weights[T*top_k + t] = sigmoid(logits[t, 0]).
+// Shared-gate only (no routed experts): weights[T*top_k + t] = sigmoid(logits[t, 0]); with
+// `routed`, the routed weights are copied in front of the gates in the same launch.
 namespace {
-__global__ void shared_gate_sigmoid_kernel(const float* __restrict__ logits, int T, int top_k,
+__global__ void shared_gate_sigmoid_kernel(const float* __restrict__ logits,
+                                           const float* __restrict__ routed, int T, int top_k,
                                            float* __restrict__ weights) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= T) return;
-  const float g = logits[(int64_t)t * 1];
-  weights[(int64_t)T * top_k + t] = 1.0f / (1.0f + expf(-g));
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t n = (int64_t)T * top_k;
+  if (routed && i < n) weights[i] = routed[i];
+  if (i < T) weights[n + i] = 1.0f / (1.0f + expf(-logits[i]));
 }
 }  // namespace
 
 hipError_t launch_shared_gate(const uint16_t* x, int T, int H, const uint16_t* shared_w,
-                              int top_k, float* logits_ws, float* weights, hipStream_t stream) {
+                              int top_k, float* logits_ws, const float* routed, float* weights,
+                              hipStream_t stream) {
   // E = 0 rows of router weight; row 0 is the shared gate. logits stride is E + 1 = 1.
   hipError_t err = launch_router_logits(x, T, H, nullptr, 0, shared_w, nullptr, logits_ws, stream);
   if (err != hipSuccess) return err;
   if (T == 0) return hipSuccess;
-  hipLaunchKernelGGL(shared_gate_sigmoid_kernel, dim3((T + 255) / 256), dim3(256), 0, stream,
-                     logits_ws, T, top_k, weights);
+  const int64_t n = routed ? (int64_t)T * top_k : T;
+  hipLaunchKernelGGL(shared_gate_sigmoid_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                     stream, logits_ws, routed, T, top_k, weights);
   return hipGetLastError();
 }

@@ -133,6 +133,43 @@ def test_fused_experts_and_moe_tokens_api():
         block.moe_tokens(x.cuda().view(2, 3, 512), torch.full((2, 3, k), 99), torch.from_numpy(w).view(2, 3, k))
 
 
+@pytest.mark.parametrize("T", [1, 2, 3, 8, 9, 40])  # slot grid, token-sum and aligned forms
+@pytest.mark.parametrize("path", ["decode", "prefill"])
+@pytest.mark.parametrize("with_shared", [False, True])
+@pytest.mark.parametrize("aliased", [False, True])
+def test_given_routing_is_read_in_place(T, path, with_shared, aliased):
+    """fused_experts on a layer call's own routing gives that call's output bit for bit and leaves
+    the routing as it was; arrays inside the output buffer are copied before it is written."""
+    import ctypes
+
+    from mtp_amd import _lib
+    _say(f"given routing T={T} {path} shared={with_shared} aliased={aliased}")
+    g = to_gpu(small_layer(3, shared=True))
+    sh = dict(shared=g.shared, shared_gate_w=g.shared_gate_w) if with_shared else {}
+    x, k = synth.make_tokens(T, 512, seed=T).cuda(), 4
+    want, ids, w = ops.moe_layer(x, g.router_w, g.experts, top_k=k, path=path, return_routing=True,
+                                 **sh)
+    if not aliased:
+        ids0, w0 = ids.clone(), w.clone()
+        assert torch.equal(ops.fused_experts(x, ids, w, g.experts, path=path, **sh), want)
+        assert torch.equal(ids, ids0) and torch.equal(w, w0)
+        return
+    out = torch.empty_like(x)  # T * k * 8 bytes of routing at the start of T * 1024 of output
+    flat, n = out.view(torch.int32).view(-1), T * k
+    flat[:n] = ids.view(-1)
+    flat[n:2 * n] = w.view(-1).view(torch.int32)
+    lib, p = _lib.load(), {"decode": 1, "prefill": 2}[path]
+    ws = torch.empty(ops.workspace_bytes(T, k, g.experts, with_shared, p), dtype=torch.uint8,
+                     device="cuda")
+    ex, shs = g.experts.struct(), g.shared.struct()
+    _lib.check(lib.moe_fused_experts_v1(
+        x.data_ptr(), T, flat.data_ptr(), flat[n:].data_ptr(), k, ctypes.byref(ex),
+        ctypes.byref(shs) if with_shared else None,
+        g.shared_gate_w.data_ptr() if with_shared else None, ws.data_ptr(), ws.numel(),
+        out.data_ptr(), p, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert torch.equal(out, want)
+
+
 def test_empty_batch_gives_empty_outputs():
     """A batch of no tokens is a no-op of every layer entry point (T = 0 returns at once; align
     writes only ntpp = 0 and takes NULL tables); the shapes come back empty."""
