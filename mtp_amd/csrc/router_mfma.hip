@@ -13,10 +13,12 @@
 //     the top-k is taken among them with the tie rule, so ids, their order and the
 //     renormalised weights are exactly those of the canonical logits.
 //
-// The bound: with S = sum_i |x_i w_i| <= |x|_2 |w_e|_2 (Cauchy-Schwarz), every fp32 summation
-// of the n = H exact bf16 x bf16 products in any order, each addition rounded with relative
-// error at most 2u (u = 2^-24; RNE gives u, the factor 2 covers a truncating accumulator), is
-// within gamma(2u, n) S of the exact sum, gamma(v, n) = n v / (1 - n v); the canonical order
+// The bound: with S = sum_i |x_i w_i| <= |x|_2 |w_e|_2 (Cauchy-Schwarz), an fp32 summation of
+// exact bf16 x bf16 products that passes each through at most n additions, each with an error of
+// at most 2u (u = 2^-24; RNE gives u, the factor 2 covers a truncating accumulator) of the sum of
+// magnitudes, is within gamma(2u, n) S of the exact sum, gamma(v, n) = n v / (1 - n v). m is
+// the sum of four partial sums over H / 4 products each, in MFMAs of 32 products and the
+// accumulator (33 terms in any order): n = 33/32 H / 4 + 3. The canonical order
 // (at most 40 roundings per product) is within gamma(u, 40) S. Adding the fp32 bias rounds each
 // side once more (<= 2u |m|), and the norms themselves are fp32 (relative error below 1e-3,
 // covered by the factor 1.01). Non-finite values make every expert a candidate.
@@ -212,54 +214,209 @@ __global__ __launch_bounds__(64 * kKSplit) void router_mfma_kernel(
   }
 }
 
-constexpr int kCertWaves = 4;
-constexpr int kCertBatch = 8;  // canonical dots whose loads are in flight together
+// The same for batches with more 32 x 64 tiles than CUs: 64 x 64 tiles whose stages all four waves
+// share, each wave 32 tokens x 32 experts (2 x 2 MFMA tiles) over the whole of K. The operand traffic
+// out of L2, T E H (1 / TT + 1 / TE) * 2 bytes, bounds these kernels (11-18 bytes a cycle and CU),
+// so the larger tile's one round of workgroups replaces two: 8192 tokens 40 -> 25 us, 4096 tokens
+// 21 -> 17 us. (64 x 128 tiles read a quarter less again but leave one workgroup per CU: 31 us at
+// 8192 tokens.) Per step one 64-k stage of 128 rows, filled as above, in a ring of four
+// stage objects with three in flight; the wait covers the wave's own loads of the step, the
+// barrier the other waves', and frees the stage that the step refills. Step s adds to
+// accumulator set s % 4, so no sum runs over more than a quarter of K (as in the K-split
+// kernel: the bound of the certificate relies on it).
+constexpr int kWideT = 64, kWideE = 64;
+__global__ __launch_bounds__(256) void router_mfma_wide_kernel(
+    const uint16_t* __restrict__ x, int T, int H, const uint16_t* __restrict__ W, int E,
+    const float* __restrict__ bias, float* __restrict__ approx, float* __restrict__ nw2) {
+  constexpr int TT = kWideT, TE = kWideE;
+  constexpr int kRows = TT + TE, kLoads = kRows / 32;  // 1 KB loads per wave and stage
+  constexpr int NE = TE / 32;                          // expert tiles per wave
+  __shared__ __attribute__((aligned(16))) uint16_t st0[kRows * kStepK];
+  __shared__ __attribute__((aligned(16))) uint16_t st1[kRows * kStepK];
+  __shared__ __attribute__((aligned(16))) uint16_t st2[kRows * kStepK];
+  __shared__ __attribute__((aligned(16))) uint16_t st3[kRows * kStepK];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // the expert tiles of a token tile share one XCD's L2, as above
+  const int tiles_e = (E + TE - 1) / TE;
+  const int n_tiles = ((T + TT - 1) / TT) * tiles_e;
+  const int chunk = (n_tiles + 7) / 8;
+  const int idx = (int)(blockIdx.x % 8) * chunk + (int)(blockIdx.x / 8);
+  if (idx >= n_tiles) return;  // workgroup-uniform
+  const int tt = idx / tiles_e, te = idx % tiles_e;
+  const int t0 = tt * TT, e0 = te * TE;
+  const __amdgpu_buffer_rsrc_t xr = buf_rsrc(x, (uint32_t)T * (uint32_t)H * 2u);
+  const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W, (uint32_t)E * (uint32_t)H * 2u);
+  const int r = lane & 15, kq = lane >> 4;
+  const int wt = wv >> 1, we = wv & 1;
+  const int steps = H / kStepK;  // H % 512 == 0: a multiple of 8
 
-// Canonical logits (routing.h:logits_tile order, bias added) of up to kCertBatch rows of W
-// (row E = the shared gate row sw) against the token chunks xc held by this lane (chunk
-// lane + 64 j); ids past n are skipped. Lane 0 writes them to out[id].
-template <int NJ>
-MOE_DEV void canonical_batch(const u32x4 (&xc)[NJ], int nq, const int* ids, int n,
-                             __amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t sr, int H, int E,
-                             const float* __restrict__ bias, float* out, int lane) {
-  u32x4 wc[kCertBatch][NJ];
+  // Load u of wave wv: 1 KB run q = wv * kLoads + u (rows 8 q .. 8 q + 7), as in the kernel above.
+  uint32_t off[kLoads];
 #pragma unroll
-  for (int b = 0; b < kCertBatch; ++b) {
-    const int e = b < n ? ids[b] : -1;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int q = lane + 64 * j;
-      const bool ok = e >= 0 && q < nq;
-      const uint32_t off = ok ? ((e == E ? 0u : (uint32_t)e * (uint32_t)H) + 8u * (uint32_t)q) * 2u
-                              : kOutOfRange;
-      wc[b][j] = buf_ld128(e == E ? sr : wr, off);
-    }
+  for (int u = 0; u < kLoads; ++u) {
+    const int R = 8 * (wv * kLoads + u) + (lane >> 3);
+    const uint32_t c = (uint32_t)((lane & 7) ^ ((R & 7) ^ ((R >> 3) & 1)));
+    const int t = t0 + R, e = e0 + R - TT;
+    const bool ok = R < TT ? t < T : e < E;
+    off[u] = ok ? ((uint32_t)(R < TT ? t : e) * (uint32_t)H + 8u * c) * 2u : kOutOfRange;
   }
+  auto dma = [&](uint16_t* st, int s) {  // a step past K loads nothing (zeros, unused)
+    const uint32_t so = s < steps ? (uint32_t)(s * kStepK * 2) : kOutOfRange;
 #pragma unroll
-  for (int b = 0; b < kCertBatch; ++b) {
-    if (b >= n) break;  // wave-uniform
-    float acc = 0.0f;
+    for (int u = 0; u < kLoads; ++u) {
+      const int q = wv * kLoads + u;  // wave-uniform; TT / 8 runs of tokens come first
+      buf_ld128_lds(q < TT / 8 ? xr : wr, st + q * 8 * kStepK, off[u] + so);
+    }
+  };
+
+  const bool norms = tt == 0 && wt == 0;  // wave-uniform
+  float n2[NE];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      if (lane + 64 * j >= nq) continue;  // no arithmetic past H (the fma chain stays exact)
+  for (int j = 0; j < NE; ++j) n2[j] = 0.0f;
+  f32x4 acc[4][2][NE];
 #pragma unroll
-      for (int el = 0; el < 8; ++el) {
-        const uint32_t xd = xc[j][el >> 1], wd = wc[b][j][el >> 1];
-        const float xf = (el & 1) ? bf16hi_to_f32(xd) : bf16lo_to_f32(xd);
-        const float wf = (el & 1) ? bf16hi_to_f32(wd) : bf16lo_to_f32(wd);
-        acc = __builtin_fmaf(xf, wf, acc);
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < NE; ++j) acc[a][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto step = [&](const uint16_t* st, uint16_t* refill, int s, f32x4(&ac)[2][NE]) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * kLoads));  // steps s + 1, s + 2 stay in flight
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of `refill` are done
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    dma(refill, s + 3);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 a[2][2], b[NE][2];  // [subtile][k-slice]
+#pragma unroll
+    for (int S = 0; S < 2; ++S) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        a[i][S] = *reinterpret_cast<const u32x4*>(
+            st + stage_chunk(32 * wt + 16 * i + r, 4 * S + kq));
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+        b[j][S] = *reinterpret_cast<const u32x4*>(
+            st + stage_chunk(TT + (TE / 2) * we + 16 * j + r, 4 * S + kq));
+    }
+#pragma unroll
+    for (int S = 0; S < 2; ++S)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NE; ++j)
+          ac[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[i][S]),
+                                                             as_bf16x8(b[j][S]), ac[i][j], 0, 0, 0);
+    if (norms) {
+#pragma unroll
+      for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int S = 0; S < 2; ++S)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            const float lo = bf16lo_to_f32(b[j][S][d]), hi = bf16hi_to_f32(b[j][S][d]);
+            n2[j] = __builtin_fmaf(lo, lo, n2[j]);
+            n2[j] = __builtin_fmaf(hi, hi, n2[j]);
+          }
+    }
+  };
+  dma(st0, 0);
+  __builtin_amdgcn_sched_barrier(0);  // issue order = step order
+  dma(st1, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  dma(st2, 2);
+  for (int s = 0; s < steps; s += 4) {
+    step(st0, st3, s, acc[0]);
+    step(st1, st0, s + 1, acc[1]);
+    step(st2, st1, s + 2, acc[2]);
+    step(st3, st2, s + 3, acc[3]);
+  }
+
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
+    const int e = e0 + (TE / 2) * we + 16 * j + r;
+    const float be = (bias && e < E) ? bias[e] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f32x4 v = (acc[0][i][j] + acc[1][i][j]) + (acc[2][i][j] + acc[3][i][j]);
+#pragma unroll
+      for (int el = 0; el < 4; ++el) {
+        const int t = t0 + 32 * wt + 16 * i + 4 * kq + el;
+        if (t < T && e < E) approx[(int64_t)t * (E + 1) + e] = v[el] + be;
       }
     }
-    acc = bfly_sum(acc);
-    const int e = ids[b];
-    if (bias && e < E) acc = acc + bias[e];
-    if (lane == 0) out[e] = acc;
+    if (norms) {
+      float v = n2[j];
+      v += xor_partner<16>(v);
+      v += xor_partner<32>(v);
+      if (kq == 0 && e < E) nw2[e] = v;
+    }
   }
 }
 
-// One wave per token. MAXC: E <= 64 MAXC; NJ: H <= 512 NJ.
+constexpr int kCertWaves = 4;
+// Canonical dots whose loads are in flight together: the first batch of a token (its top-k), and
+// the following ones (a shared gate, near-ties).
+constexpr int kCertBatch = 8, kCertRest = 2;
+
+// Canonical logits (routing.h:logits_tile order, bias added) of the n <= B rows ids[0 .. n) of W
+// (row E = the shared gate row sr) against the token's chunks xc held by this lane (chunk
+// lane + 64 j, H == 512 NJ), written to out[id]. The rows' chunks j and j + 1 are in flight at a
+// time (all four at once: 183 VGPRs, two waves per SIMD instead of four), a token's chunk is
+// widened once for all rows, and the lanes' partials are added by the transposed butterfly: with
+// the tighter bound of the certificate, 51.7 -> 33.7 us at 8192 tokens, 14.2 -> 11.6 us at 2048 (hidden
+// 2048, 256 experts). What is left is the rows' traffic out of L2, 32 KB per token. (A ring of four
+// rows with a row's load behind each sum: 56.7 and 19.9 us.)
+template <int B, int NJ>
+MOE_DEV void canonical_batch(const u32x4 (&xc)[NJ], const int* ids, int n,
+                             __amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t sr, int H, int E,
+                             const float* __restrict__ bias, float* out, int lane) {
+  int e[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) e[b] = __builtin_amdgcn_readfirstlane(b < n ? ids[b] : -1);
+  u32x4 wc[2][B];
+  auto load = [&](int slot, int j) {  // a row past n reads zeros without a memory access
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const uint32_t ro = e[b] < 0 ? kOutOfRange : (e[b] == E ? 0u : (uint32_t)e[b] * (uint32_t)H * 2u);
+      wc[slot][b] = buf_ld128(e[b] == E ? sr : wr, ro + 16u * (uint32_t)(lane + 64 * j));
+    }
+  };
+  load(0, 0);
+  if (NJ > 1) load(1, 1);
+  float acc[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) acc[b] = 0.0f;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    __builtin_amdgcn_sched_barrier(0);  // the loads of chunk j + 1 before the wait for chunk j
+#pragma unroll
+    for (int el = 0; el < 8; ++el) {
+      const uint32_t xd = xc[j][el >> 1];
+      const float xf = (el & 1) ? bf16hi_to_f32(xd) : bf16lo_to_f32(xd);
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const uint32_t wd = wc[j & 1][b][el >> 1];
+        acc[b] = __builtin_fmaf(xf, (el & 1) ? bf16hi_to_f32(wd) : bf16lo_to_f32(wd), acc[b]);
+      }
+    }
+    if (j + 2 < NJ) load(j & 1, j + 2);
+  }
+  fold_partials(acc, lane);
+  const int v = lane / (64 / B);  // the row whose sum this lane holds
+  if (lane % (64 / B) == 0 && v < n) {
+    const int id = ids[v];
+    out[id] = bias && id < E ? acc[0] + bias[id] : acc[0];
+  }
+}
+
+// One wave per token. MAXC: E <= 64 MAXC; H == 512 NJ.
 template <int MAXC, int NJ>
-__global__ __launch_bounds__(64 * kCertWaves) void router_certify_kernel(
+__global__ __launch_bounds__(64 * kCertWaves, MAXC == 4 ? 4 : 3) void router_certify_kernel(
     const uint16_t* __restrict__ x, int T, int H, const uint16_t* __restrict__ W, int E,
     const uint16_t* __restrict__ shared_w, const float* __restrict__ bias,
     const float* __restrict__ approx, const float* __restrict__ nw2, float rel_bound, int top_k,
@@ -348,9 +505,10 @@ __global__ __launch_bounds__(64 * kCertWaves) void router_certify_kernel(
 
   const __amdgpu_buffer_rsrc_t wr = buf_rsrc(W, (uint32_t)E * (uint32_t)H * 2u);
   const __amdgpu_buffer_rsrc_t sr = buf_rsrc(shared_w, has_shared ? (uint32_t)H * 2u : 0u);
-  for (int b0 = 0; b0 < n_dots; b0 += kCertBatch)
-    canonical_batch<NJ>(xc, nq, list + b0, min(kCertBatch, n_dots - b0), wr, sr, H, E, bias,
-                        exact, lane);
+  canonical_batch<kCertBatch>(xc, list, min(kCertBatch, n_dots), wr, sr, H, E, bias, exact, lane);
+  for (int b0 = kCertBatch; b0 < n_dots; b0 += kCertRest)
+    canonical_batch<kCertRest>(xc, list + b0, min(kCertRest, n_dots - b0), wr, sr, H, E, bias,
+                               exact, lane);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -412,16 +570,21 @@ hipError_t launch_certify(const uint16_t* x, int T, int H, const uint16_t* W, in
 
 }  // namespace
 
+constexpr int kCus = 256;
+
 bool router_prefill_fits(int T, int H, int E, int top_k) {
   return T >= 1 && H >= 512 && H <= 2048 && H % 512 == 0 && E >= 1 && E <= 512 && top_k >= 1 &&
          top_k <= 64 && top_k <= E && (int64_t)T * H * 2 < kOutOfRange &&
          (int64_t)E * H * 2 < kOutOfRange;
 }
 
-// Relative bound factor: gamma(2u, H) + gamma(u, 40), times 1.01 for the fp32 norms.
+// Relative bound factor: gamma(2u, 33/32 H / 4 + 3) + gamma(u, 40), times 1.01 for the fp32
+// norms. (With n = H, as if one sum ran over all of K, four times as many experts lie within the
+// bound of the k-th logit, and a token with one of them needs a second batch of canonical dots.)
 float router_prefill_rel_bound(int H) {
   const double u = 1.0 / 16777216.0;
-  const double g_any = (2.0 * u * H) / (1.0 - 2.0 * u * H);
+  const double n = 33.0 / 32.0 * H / 4.0 + 3.0;
+  const double g_any = (2.0 * u * n) / (1.0 - 2.0 * u * n);
   const double g_can = (u * 40.0) / (1.0 - u * 40.0);
   return (float)((g_any + g_can) * 1.01);
 }
@@ -431,10 +594,16 @@ hipError_t launch_router_prefill(const uint16_t* x, int T, int H, const uint16_t
                                  float* approx, float* nw2, int32_t* ids, float* weights,
                                  hipStream_t stream) {
   if (!router_prefill_fits(T, H, E, top_k)) return hipErrorInvalidValue;
-  const int tiles = ((T + kTileT - 1) / kTileT) * ((E + kTileE - 1) / kTileE);
-  hipLaunchKernelGGL(router_mfma_kernel, dim3((tiles + 7) / 8 * 8), dim3(64 * kKSplit), 0, stream,
-                     x, T, H, W, E, bias, approx, nw2);
-  hipError_t err = hipGetLastError();
+  auto mfma = [&](auto kernel, int tt, int te) {
+    const int tiles = ((T + tt - 1) / tt) * ((E + te - 1) / te);
+    hipLaunchKernelGGL(kernel, dim3((tiles + 7) / 8 * 8), dim3(256), 0, stream, x, T, H, W, E, bias,
+                       approx, nw2);
+    return hipGetLastError();
+  };
+  // the small tiles while each has a CU of its own (2048 tokens of 256 experts: 10.5 us)
+  const int64_t small = (int64_t)((T + kTileT - 1) / kTileT) * ((E + kTileE - 1) / kTileE);
+  hipError_t err = small <= kCus ? mfma(router_mfma_kernel, kTileT, kTileE)
+                                 : mfma(router_mfma_wide_kernel, kWideT, kWideE);
   if (err != hipSuccess) return err;
   const float rel = router_prefill_rel_bound(H);
   const int nj = H / 512;

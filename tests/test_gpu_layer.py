@@ -133,6 +133,28 @@ def test_fused_experts_and_moe_tokens_api():
         block.moe_tokens(x.cuda().view(2, 3, 512), torch.full((2, 3, k), 99), torch.from_numpy(w).view(2, 3, k))
 
 
+# (T, E, H): both router tile shapes (32 x 64, and 64 x 64 from 256 tiles on) with token
+# and expert counts that end inside a tile, at the fewest and at other numbers of 64-k steps
+@pytest.mark.parametrize("T,E,H", [(333, 300, 512), (1061, 512, 512), (1700, 300, 1536),
+                                   (2090, 512, 1024), (3300, 300, 512)])
+def test_prefill_router_tiles_match_the_canonical_router(T, E, H):
+    """Routing of the prefill path's tiles: ids and weights are the canonical router's bit for bit,
+    with exact ties across experts and rows of equal logits among the tokens."""
+    _say(f"prefill router tiles T={T} E={E} H={H}")
+    g = synth.make_layer(11, num_experts=E, hidden=H, intermediate=256, zipf=True, shared=True,
+                         device="cuda")
+    x = synth.make_tokens(T, H, seed=5).cuda()
+    rw = g.router_w.clone()
+    rw[E - 1], rw[3] = rw[0], rw[2]
+    bias = g.logit_bias.clone()
+    bias[E - 1], bias[3] = bias[0], bias[2]
+    x[T - 1] = 0
+    _, ids, w = ops.moe_layer(x, rw, g.experts, top_k=8, logit_bias=bias, shared=g.shared,
+                              shared_gate_w=g.shared_gate_w, path="prefill", return_routing=True)
+    r_ids, r_w, _, _ = ops.router_topk(x, rw, 8, logit_bias=bias, shared_gate_w=g.shared_gate_w)
+    assert torch.equal(ids, r_ids) and torch.equal(w, r_w)
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 8, 9, 40])  # slot grid, token-sum and aligned forms
 @pytest.mark.parametrize("path", ["decode", "prefill"])
 @pytest.mark.parametrize("with_shared", [False, True])
