@@ -4,10 +4,10 @@
 // known-answer test is tests/test_vllm_descriptor_mapping_assertion.py:1012-1085).
 //
 // Decode sizes: one workgroup of 16 waves (routing.h:align_block). Wave w owns a contiguous
-// range of slots. Pass 1 builds per-wave expert histograms in LDS; pass 2 turns them into
-// exclusive per-(wave, expert) base positions; pass 3 walks each range 64 slots at a time in slot
-// order, ranks equal experts inside the wave with a ballot-based match, and scatters. The order
-// is therefore experts ascending, slots ascending within an expert - a stable argsort.
+// range of slots. It ranks equal experts inside its range 64 slots at a time in slot order with a
+// ballot-based match, which leaves its per-expert counts in LDS; the counts become exclusive
+// per-(wave, expert) base positions, and every slot goes to base + rank. The order is therefore
+// experts ascending, slots ascending within an expert - a stable argsort.
 // Large inputs (prefill): the same ranking per chunk in many single-wave workgroups, then one
 // block for the offsets and the scatter (align_chunk_kernel / align_finish_kernel below).
 #include "launch.h"
@@ -52,13 +52,7 @@ __global__ __launch_bounds__(64) void align_chunk_kernel(const int32_t* __restri
       if (base0 + 64 * u >= hi) break;  // uniform
       const int e = eb[u];
       const bool valid = e >= 0;
-      uint64_t peers = __ballot(valid);
-#pragma unroll
-      for (int bit = 0; bit < 10; ++bit) {
-        const bool b = valid && ((e >> bit) & 1);
-        const uint64_t bal = __ballot(b);
-        peers &= b ? bal : ~bal;
-      }
+      const uint64_t peers = expert_peers(e);
       if (valid) scratch[f] = cnt[e] + __popcll(peers & lt_mask);
       __builtin_amdgcn_wave_barrier();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -127,10 +121,10 @@ __global__ __launch_bounds__(1024) void align_kernel(const int32_t* __restrict__
                                                      int cap, int32_t* __restrict__ sorted,
                                                      int32_t* __restrict__ eids,
                                                      int32_t* __restrict__ ntpp,
-                                                     int32_t* __restrict__ border) {
+                                                     int32_t* __restrict__ border, bool fill_tail) {
   __shared__ AlignSmem sm;
   __shared__ int s_wtot[kOrderMaxClasses][16];
-  align_block(topk_ids, T, top_k, E, has_shared, BM, cap, sorted, eids, ntpp, sm);
+  align_block(topk_ids, T, top_k, E, has_shared, BM, cap, sorted, eids, ntpp, sm, fill_tail);
   if (border) {
     __syncthreads();  // every wave's scatter is done with its counters
     const int G = E + (has_shared ? 1 : 0);
@@ -383,7 +377,7 @@ int64_t align_scratch_bytes(int T, int top_k, int E, int has_shared, int BM, int
 
 hipError_t launch_align(const int32_t* topk_ids, int T, int top_k, int E, int has_shared, int BM,
                         int cap, int32_t* sorted, int32_t* eids, int32_t* ntpp, int32_t* border,
-                        int32_t* scratch, hipStream_t stream) {
+                        int32_t* scratch, bool fill_tail, hipStream_t stream) {
   int CH = 0;
   const int nchunks = align_chunks(T, top_k, E, has_shared, BM, cap, scratch != nullptr, &CH);
   if (nchunks > 0 && scratch) {
@@ -407,6 +401,6 @@ hipError_t launch_align(const int32_t* topk_ids, int T, int top_k, int E, int ha
   }
   hipLaunchKernelGGL(align_kernel, dim3(1), dim3(1024), 0, stream, topk_ids, T, top_k, E,
                      has_shared, BM, cap, sorted, eids, ntpp,
-                     (BM % 16 == 0 && BM <= 16 * kOrderMaxClasses) ? border : nullptr);
+                     (BM % 16 == 0 && BM <= 16 * kOrderMaxClasses) ? border : nullptr, fill_tail);
   return hipGetLastError();
 }

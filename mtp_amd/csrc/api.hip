@@ -202,7 +202,7 @@ int run_experts(const uint16_t* x, int T, int top_k, const moe_expert_set_v1* ex
   } else {
     if (routing == ROUTE_ALIGN) {
       MOE_CHECK_HIP(launch_align(ids, T, top_k, ex->num_experts, has_shared, L.bm, L.cap, sorted,
-                                 eids, ntpp, border, scratch, stream), "align");
+                                 eids, ntpp, border, scratch, false, stream), "align");
     }
     MOE_CHECK_HIP(dispatch_w1(path, x, ed, sd, sorted, eids, ntpp, border, L.bm, L.cap, h, stream),
                   "w1");
@@ -367,7 +367,7 @@ int moe_align_v1(const int32_t* topk_ids, int32_t T, int32_t top_k, int32_t num_
                 need);
   MOE_CHECK_HIP(launch_align(topk_ids, T, top_k, num_experts, has_shared ? 1 : 0, block_m,
                              capacity_blocks, sorted_ids, expert_ids, ntpp, nullptr, nullptr,
-                             (hipStream_t)stream),
+                             true, (hipStream_t)stream),
                 "align");
   return MOE_OK;
 }

@@ -82,10 +82,11 @@ int align_capacity_blocks(int T, int top_k, int E, int has_shared, int BM);
 int64_t align_scratch_bytes(int T, int top_k, int E, int has_shared, int BM, int cap);
 // scratch (nullable): align_scratch_bytes bytes the call may overwrite. Without it, inputs of up to
 // 32 768 slots still take a two-kernel form (ranks and counts in the sorted buffer), larger ones the
-// one-block kernel.
+// one-block kernel. fill_tail false lets the one-block kernel leave the entries past the padded
+// total unwritten (every GEMM block checks ntpp before it uses them).
 hipError_t launch_align(const int32_t* topk_ids, int T, int top_k, int E, int has_shared, int BM,
                         int cap, int32_t* sorted, int32_t* eids, int32_t* ntpp, int32_t* border,
-                        int32_t* scratch, hipStream_t stream);
+                        int32_t* scratch, bool fill_tail, hipStream_t stream);
 
 // Slot-grid routing for decode-size batches (slot_grid_fits): the MFMA decode kernels take their
 // expert and rows from the routed ids themselves instead of an align pass. Workgroup y = slot

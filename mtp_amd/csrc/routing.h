@@ -456,57 +456,108 @@ MOE_DEV void align_ids(__amdgpu_buffer_rsrc_t ir, int routed, int E, int base, i
   }
 }
 
-// topk_ids in global memory.
+// Slots of a 64-slot chunk with this lane's expert (e < 0: no slot), from one ballot per id bit.
+MOE_DEV uint64_t expert_peers(int e) {
+  const bool valid = e >= 0;
+  uint64_t peers = __ballot(valid);
+#pragma unroll
+  for (int bit = 0; bit < 10; ++bit) {
+    const bool b = valid && ((e >> bit) & 1);
+    const uint64_t bal = __ballot(b);
+    peers &= b ? bal : ~bal;
+  }
+  return peers;
+}
+
+// topk_ids in global memory. One workgroup, so what bounds it is its chain of dependent steps.
+// Up to kAlignIds chunks of 64 slots per wave (8192 slots) a wave's ids stay in registers from the
+// one load on: the ballot match ranks a chunk's slots and leaves the wave's counts behind, one
+// pass over the groups turns the counts into bases, and the slots, the padding and the block ids
+// are stored together after the last barrier (a barrier between stores waits for the earlier
+// ones). Against counting with LDS atomics, loading the ids a second time and ranking them after
+// the padding's stores: eight layers of 48 tokens (64 experts, top-4) 168.5 -> 163.5 us, of 64
+// tokens (256 experts, top-8) 524 -> 514 us; one layer of 203 tokens 98.7 -> 97.7 us. Larger
+// inputs keep that form: their ids do not fit the registers.
+// With fill_tail false the entries past the padded total are left as they are, as in align_wave.
 MOE_DEV void align_block(const int32_t* topk_ids, int T, int top_k, int E, int has_shared, int BM,
                          int cap, int32_t* __restrict__ sorted, int32_t* __restrict__ eids,
-                         int32_t* __restrict__ ntpp, AlignSmem& sm) {
+                         int32_t* __restrict__ ntpp, AlignSmem& sm, bool fill_tail) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int routed = T * top_k;
   const int n_slots = routed + (has_shared ? T : 0);
   const int G = E + (has_shared ? 1 : 0);
   const BlockDiv bd(BM);
-  for (int i = tid; i < kAlignWaves * kMaxGroups; i += 1024) (&sm.cnt[0][0])[i] = 0;
-  __syncthreads();
-
   const int per_wave = (((n_slots + kAlignWaves - 1) / kAlignWaves) + 63) / 64 * 64;
   const int lo = min(w * per_wave, n_slots), hi = min(lo + per_wave, n_slots);
+  const bool held = per_wave <= 64 * kAlignIds;  // uniform over the workgroup
   const __amdgpu_buffer_rsrc_t ir = buf_rsrc(topk_ids, (uint32_t)routed * 4u);
-  for (int base = lo; base < hi; base += 64 * kAlignIds) {
-    int e[kAlignIds];
-    align_ids(ir, routed, E, base, hi, lane, e);
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int eb[kAlignIds], rank[kAlignIds];
+  align_ids(ir, routed, E, lo, hi, lane, eb);
+  // every wave clears and fills its own counters: LDS operations of one wave complete in order
+  for (int g = lane; g < G; g += 64) sm.cnt[w][g] = 0;
+  __builtin_amdgcn_wave_barrier();
+  if (held) {
 #pragma unroll
     for (int u = 0; u < kAlignIds; ++u) {
-      if (base + 64 * u >= hi) break;  // uniform
-      if (e[u] >= 0) atomicAdd(&sm.cnt[w][e[u]], 1);
+      if (lo + 64 * u >= hi) break;  // uniform over the wave
+      const int e = eb[u];
+      const uint64_t peers = expert_peers(e);
+      const int before = (u > 0 && e >= 0) ? sm.cnt[w][e] : 0;
+      rank[u] = before + __popcll(peers & lt_mask);
+      __builtin_amdgcn_wave_barrier();  // every lane has read the old count
+      if (e >= 0 && (peers & lt_mask) == 0) sm.cnt[w][e] = before + __popcll(peers);
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else {
+    for (int base = lo; base < hi; base += 64 * kAlignIds) {
+      int e[kAlignIds];
+      align_ids(ir, routed, E, base, hi, lane, e);
+#pragma unroll
+      for (int u = 0; u < kAlignIds; ++u) {
+        if (base + 64 * u >= hi) break;  // uniform
+        if (e[u] >= 0) atomicAdd(&sm.cnt[w][e[u]], 1);
+      }
     }
   }
   __syncthreads();
+  // Thread g: group g's size, the exclusive scan of the padded sizes over the groups, and the
+  // waves' bases in place of their counts; pad[] keeps the end of the group's real slots.
   int tp;
-  {  // padded group sizes and their exclusive scan over the groups (thread g: group g)
-    int tot = 0;
-    if (tid < G)
-      for (int v = 0; v < kAlignWaves; ++v) tot += sm.cnt[v][tid];
-    const int pad = bd.pad(tot);
-    if (tid < G) sm.pad[tid] = pad;
-    const int off = block_excl_sum(pad, sm.wtot, tp);
-    if (tid < G) sm.off[tid] = off;
-  }
-  __syncthreads();
-  // Bases: one thread per group turns the 16 waves' counts into running offsets (all groups in
-  // parallel) and leaves the end of the group's real slots in pad[]. Then four threads per group
-  // write its padding sentinels with 16-byte stores (scalar stores for an unaligned head or tail)
-  // and its block ids; a group's padded end is the next group's offset.
-  const int limit = cap * BM;
-  for (int g = tid; g < G; g += 1024) {
-    int run = sm.off[g];
+  {
+    int c[kAlignWaves], tot = 0;
+#pragma unroll
     for (int v = 0; v < kAlignWaves; ++v) {
-      const int c = sm.cnt[v][g];
-      sm.cnt[v][g] = run;
-      run += c;
+      c[v] = tid < G ? sm.cnt[v][tid] : 0;
+      tot += c[v];
     }
-    sm.pad[g] = run;
+    const int off = block_excl_sum(bd.pad(tot), sm.wtot, tp);
+    if (tid < G) {
+      sm.off[tid] = off;
+      sm.pad[tid] = off + tot;
+      int run = off;
+#pragma unroll
+      for (int v = 0; v < kAlignWaves; ++v) {
+        sm.cnt[v][tid] = run;
+        run += c[v];
+      }
+    }
   }
   __syncthreads();
+  const int limit = cap * BM;
+  // Stable scatter: ranges in wave order, slots in order inside a range.
+  if (held) {
+#pragma unroll
+    for (int u = 0; u < kAlignIds; ++u) {
+      if (lo + 64 * u >= hi) break;  // uniform over the wave
+      if (eb[u] >= 0) {
+        const int pos = sm.cnt[w][eb[u]] + rank[u];
+        if (pos < limit) sorted[pos] = lo + 64 * u + lane;
+      }
+    }
+  }
+  // Four threads per group write its padding sentinels with 16-byte stores (scalar stores for an
+  // unaligned head or tail) and its block ids; a group's padded end is the next group's offset.
   const bool vec = (reinterpret_cast<uintptr_t>(sorted) & 15u) == 0;
   for (int g = tid >> 2; g < G; g += 256) {
     const int sub = tid & 3;
@@ -524,38 +575,28 @@ MOE_DEV void align_block(const int32_t* topk_ids, int T, int top_k, int E, int h
     const int bend = min(bd.div(end), cap);
     for (int b = bd.div(off) + sub; b < bend; b += 4) eids[b] = g;
   }
-  for (int b = bd.div(tp) + tid; b < cap; b += 1024) eids[b] = -1;
-  for (int p = tp + tid; p < cap * BM; p += 1024) sorted[p] = n_slots;
+  if (fill_tail) {
+    for (int b = bd.div(tp) + tid; b < cap; b += 1024) eids[b] = -1;
+    for (int p = tp + tid; p < limit; p += 1024) sorted[p] = n_slots;
+  }
   if (tid == 0) *ntpp = tp;
-  __syncthreads();
+  if (held) return;
 
-  // Stable scatter: ranges in wave order, slots in order inside a range.
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   for (int base0 = lo; base0 < hi; base0 += 64 * kAlignIds) {
-    int eb[kAlignIds];
     align_ids(ir, routed, E, base0, hi, lane, eb);
 #pragma unroll
     for (int u = 0; u < kAlignIds; ++u) {
       const int base = base0 + 64 * u;
       if (base >= hi) break;  // uniform: the rest of the batch lies past the wave's range
-      const int f = base + lane;
       const int e = eb[u];
-      const bool valid = e >= 0;
-      uint64_t peers = __ballot(valid);
-#pragma unroll
-      for (int bit = 0; bit < 10; ++bit) {
-        const bool b = valid && ((e >> bit) & 1);
-        const uint64_t bal = __ballot(b);
-        peers &= b ? bal : ~bal;
-      }
-      if (valid) {
-        const int rank = __popcll(peers & lt_mask);
-        const int pos = sm.cnt[w][e] + rank;
-        if (pos < cap * BM) sorted[pos] = f;
+      const uint64_t peers = expert_peers(e);
+      if (e >= 0) {
+        const int pos = sm.cnt[w][e] + __popcll(peers & lt_mask);
+        if (pos < limit) sorted[pos] = base + lane;
       }
       // wave-local LDS update after every lane has read the old base
       __builtin_amdgcn_wave_barrier();
-      if (valid && (__ffsll((long long)peers) - 1) == lane) sm.cnt[w][e] += __popcll(peers);
+      if (e >= 0 && (peers & lt_mask) == 0) sm.cnt[w][e] += __popcll(peers);
       __builtin_amdgcn_wave_barrier();
     }
   }
@@ -579,13 +620,7 @@ MOE_DEV void align_wave(const int32_t* topk_ids, int T, int top_k, int E, int ha
   const int G = E + (has_shared ? 1 : 0);
   const int e = (lane < n_slots) ? slot_expert(topk_ids, routed, E, lane) : -1;
   const bool valid = e >= 0;
-  uint64_t peers = __ballot(valid);
-#pragma unroll
-  for (int bit = 0; bit < 10; ++bit) {
-    const bool b = valid && ((e >> bit) & 1);
-    const uint64_t bal = __ballot(b);
-    peers &= b ? bal : ~bal;
-  }
+  const uint64_t peers = expert_peers(e);
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const int rank = __popcll(peers & lt_mask);
   const int cnt = __popcll(peers);

@@ -166,6 +166,26 @@ def test_align_bit_exact(T, k, E, BM, shared, zipf):
     assert np.array_equal(s.cpu().numpy(), rs)
 
 
+@pytest.mark.parametrize("T,k,E,BM,shared", [(65, 1, 512, 16, True),  # a second chunk, 513 groups
+                                             (203, 8, 256, 16, True),
+                                             # 8192 slots: the last that the registers hold; then
+                                             # one more token
+                                             (1024, 8, 64, 16, False), (1025, 8, 64, 16, False)])
+def test_align_held_ids(T, k, E, BM, shared):
+    """The one-workgroup align with several chunks per wave, with experts that fill whole chunks
+    (every token picks expert 0)."""
+    _say(f"align held ids T={T} k={k} E={E} BM={BM} shared={shared}")
+    rng = np.random.default_rng(T)
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    ids[:, 0] = 0
+    cap = ops.capacity_blocks(T, k, E, shared, BM)
+    s, e, n = ops.align(torch.from_numpy(ids).cuda(), E, BM, has_shared=shared)
+    rs, re_, rn = moe_ref.align_block_padded(ids, E, BM, has_shared=shared, capacity_blocks=cap)
+    assert int(n.item()) == rn
+    assert np.array_equal(e.cpu().numpy(), re_)
+    assert np.array_equal(s.cpu().numpy(), rs)
+
+
 def test_align_known_answer():
     _say("align KAT")
     s, e, n = ops.align(torch.tensor([[1, 2, 3]], dtype=torch.int32).cuda(), 8, 4)
