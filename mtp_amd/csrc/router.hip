@@ -209,19 +209,21 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restric
 
 // One wave per token for the top-k, then wave 0 aligns the (at most 64) slots.
 __global__ __launch_bounds__(64 * kTopkAlignMaxTokens) void topk_align_kernel(
-    const float* __restrict__ logits, int T, int E, int top_k, int has_shared, int BM, int cap,
+    const float* __restrict__ logits, int T, int E, int top_k, int has_shared, int cap,
     int32_t* __restrict__ ids, float* __restrict__ weights, int32_t* __restrict__ sorted,
     int32_t* __restrict__ eids, int32_t* __restrict__ ntpp) {
   __shared__ int s_ids[kAlignWaveMaxSlots];
-  __shared__ int s_pad[kMaxGroups];
+  __shared__ AlignWaveSmem sm;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (wave < T)
     topk_token_any(logits + (int64_t)wave * (E + 1), E, top_k, has_shared, T, wave, lane, ids,
                weights, s_ids);
-  __syncthreads();
-  if (wave == 0)
-    align_wave(s_ids, T, top_k, E, has_shared, BM, cap, sorted, eids, ntpp, lane, s_pad,
-               false);  // internal layout: the decode kernels stop at the padded total
+  // Every wave's ids are in LDS; a barrier without __syncthreads' release fence, which would also
+  // wait for the stores of the ids and weights to memory.
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  if (wave == 0) align_wave(s_ids, T, top_k, E, has_shared, cap, sorted, eids, ntpp, lane, sm);
 }
 
 template <int TT, int TE>
@@ -289,9 +291,9 @@ hipError_t launch_router_topk(const float* logits, int T, int E, int top_k, int 
 hipError_t launch_topk_align(const float* logits, int T, int E, int top_k, int has_shared, int BM,
                              int cap, int32_t* ids, float* weights, int32_t* sorted, int32_t* eids,
                              int32_t* ntpp, hipStream_t stream) {
-  if (!topk_align_fits(T, top_k, has_shared)) return hipErrorInvalidValue;
+  if (!topk_align_fits(T, top_k, has_shared) || BM != kAlignWaveBlock) return hipErrorInvalidValue;
   hipLaunchKernelGGL(topk_align_kernel, dim3(1), dim3(64 * T), 0, stream, logits, T, E, top_k,
-                     has_shared, BM, cap, ids, weights, sorted, eids, ntpp);
+                     has_shared, cap, ids, weights, sorted, eids, ntpp);
   return hipGetLastError();
 }
 
