@@ -274,7 +274,11 @@ MOE_DEV void projections(const ExpertsDev& ed, int mode, bool is_shared, ProjDev
 }
 
 // Block = one 16-slot expert block x (16 * CT) columns; KS waves split K evenly (each slice a
-// whole number of quantisation groups) and are summed through LDS in wave order.
+// whole number of quantisation groups) and are summed through LDS in wave order. Every wave adds
+// and finishes its share of the tile (EPW of a lane's four rows x JPW of its columns): with wave 0
+// alone doing it, the sums, SiLUs and stores of the whole tile were a serial tail of each
+// workgroup (eight layers: of one token 160 -> 156 us, of 64 518 -> 508 us; of 48 with 64 experts
+// 159 -> 153 us; one layer of 203 tokens 97.4 -> 95.5 us).
 // NB > 0 and NGW == 0: runtime loop over the wave's groups with an NB-deep ring; NB < 0: a
 // slice of exactly -NB groups, all loaded up front; NGW > 0: a slice of exactly NGW groups with
 // an NB-deep ring, unrolled.
@@ -293,11 +297,17 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
   constexpr int NT = NP * CT;                    // MFMA N-subtiles per lane
   constexpr int TW = 16 * CT;                    // columns per block
   static_assert(!FW2 || (MODE == DEC_W1 && CT == 2), "fused W2: W1 blocks of 32 columns");
-  __shared__ float red[(KS > 1 ? KS - 1 : 1) * NT * 4 * 64];
+  constexpr int EPW = KS >= 4 ? 1 : 4 / KS;             // rows per lane that a wave finishes
+  constexpr int JPW = KS > 4 ? CT * 4 / KS : CT;        // columns per lane that it finishes
+  static_assert(JPW >= 1 && EPW * JPW * KS == 4 * CT, "an even share of the tile for every wave");
+  __shared__ float red[KS > 1 ? KS * NT * 4 * 64 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar K-slice offsets
-  int e, f_m, f_out[4];  // expert; A row of this lane; D rows of this lane
+  const int el0 = KS >= 4 ? wave * 4 / KS : wave * EPW;  // this wave's share of the tile
+  const int j0 = KS > 4 ? (wave % (KS / 4)) * JPW : 0;
+  constexpr int NF = FW2 ? 4 : EPW;  // fused W2: every wave writes all the rows
+  int e, f_m, f_out[NF];  // expert; A row of this lane; the D rows of this lane that it writes
   __shared__ float s_w[kSlotGridMaxSlots + kTopkAlignMaxTokens];  // slot grid: routed weights
   if (sg.active) {
     // Slot grid (SlotGrid in launch.h): slots from the routed ids, no align pass.
@@ -339,9 +349,9 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
     __syncthreads();
     f_m = (lane & 15) < cnt ? s_rows[lane & 15] : n_slots;
 #pragma unroll
-    for (int el = 0; el < 4; ++el) {
-      const int r = 4 * (lane >> 4) + el;
-      f_out[el] = r < cnt ? s_rows[r] : n_slots;
+    for (int i = 0; i < NF; ++i) {
+      const int r = 4 * (lane >> 4) + (FW2 ? 0 : el0) + i;
+      f_out[i] = r < cnt ? s_rows[r] : n_slots;
     }
     if constexpr (FW2) {
       if (!expert_ok(ed, e)) {  // dropped slots: zero partial rows for this column block
@@ -360,7 +370,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
     e = eids[b];
     f_m = sorted[b * kBM + (lane & 15)];
 #pragma unroll
-    for (int el = 0; el < 4; ++el) f_out[el] = sorted[b * kBM + 4 * (lane >> 4) + el];
+    for (int i = 0; i < NF; ++i) f_out[i] = sorted[b * kBM + 4 * (lane >> 4) + el0 + i];
     if (b * kBM >= n_padded || !expert_ok(ed, e)) return;
   }
 
@@ -412,6 +422,16 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
     __builtin_amdgcn_sched_barrier(0);  // issued here, with the W1 stream, not at their use
   }
 
+  // the rows' routed weights, in flight with the weight stream (their first use is the epilogue)
+  [[maybe_unused]] float w_out[EPW];
+  if constexpr (MODE == DEC_W2) {
+    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(topk_w, (uint32_t)sd.num_slots * 4u);
+#pragma unroll
+    for (int i = 0; i < EPW; ++i)  // a padding row's offset lies past the end: zero
+      w_out[i] = __uint_as_float(buf_ld32(wr, (uint32_t)f_out[i] * 4u));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   f32x4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -423,47 +443,53 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
     decode_tile<NP, SPG, CT, NB>(tile, acc);
   }
 
-  if constexpr (KS > 1) {  // cross-wave reduction: waves 1.. write, wave 0 sums in wave order
-    if (wave > 0) {
+  // This wave's share: out[p][i][j] = element el0 + i of N-subtile j0 + j of projection p, the
+  // waves' partial sums added in wave order.
+  float fin[NP][EPW][JPW];
+  if constexpr (KS > 1) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) red[(((wave - 1) * NT + t) * 4 + i) * 64 + lane] = acc[t][i];
-    }
+      for (int i = 0; i < 4; ++i) red[((wave * NT + t) * 4 + i) * 64 + lane] = acc[t][i];
     __syncthreads();
-    if constexpr (!FW2) {
-      if (wave != 0) return;
-      for (int w = 1; w < KS; ++w)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+    for (int p = 0; p < NP; ++p)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[t][i] += red[(((w - 1) * NT + t) * 4 + i) * 64 + lane];
-    } else if (wave == 0) {
-      for (int w = 1; w < KS; ++w)
+      for (int i = 0; i < EPW; ++i)
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int j = 0; j < JPW; ++j) {
+          const float* src = red + ((p * CT + j0 + j) * 4 + el0 + i) * 64 + lane;
+          float v = src[0];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[t][i] += red[(((w - 1) * NT + t) * 4 + i) * 64 + lane];
-    }
+          for (int w = 1; w < KS; ++w) v += src[w * NT * 4 * 64];
+          fin[p][i][j] = v;
+        }
+  } else {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int i = 0; i < EPW; ++i)
+#pragma unroll
+        for (int j = 0; j < JPW; ++j) fin[p][i][j] = acc[p * CT + j][i];
   }
 
   if constexpr (FW2) {
-    // h rows of the block (bf16, as W1 writes them) into LDS as [16 rows][16 column pairs]
-    __shared__ uint32_t s_h[kBM * 16];
-    if (wave == 0) {
+    // h rows of the block (bf16, as W1 writes them) into LDS as [16 rows][32 columns]
+    __shared__ __attribute__((aligned(16))) uint16_t s_h[kBM * TW];
 #pragma unroll
-      for (int el = 0; el < 4; ++el) {
-        const bool real = (unsigned)f_out[el] < (unsigned)sd.num_slots;
-        s_h[(4 * kq + el) * 16 + m] =
-            real ? pack_bf16x2(silu_f32(acc[0][el]) * acc[CT][el],
-                               silu_f32(acc[1][el]) * acc[CT + 1][el])
-                 : 0u;
-      }
+    for (int i = 0; i < EPW; ++i) {
+      int f = f_out[0];  // f_out[el0 + i] without an indexed register read
+#pragma unroll
+      for (int r = 1; r < NF; ++r) f = el0 + i == r ? f_out[r] : f;
+      const bool real = (unsigned)f < (unsigned)sd.num_slots;
+#pragma unroll
+      for (int j = 0; j < JPW; ++j)
+        s_h[(4 * kq + el0 + i) * TW + CT * m + j0 + j] =
+            real ? (uint16_t)f32_to_bf16_rne(silu_f32(fin[0][i][j]) * fin[1][i][j]) : 0;
     }
     __syncthreads();
     // A: row m, k 8 kq .. 8 kq + 7 of the block's 32 h columns; X[row] = sum of the row's h
-    const u32x4 hv = {s_h[m * 16 + 4 * kq], s_h[m * 16 + 4 * kq + 1], s_h[m * 16 + 4 * kq + 2],
-                      s_h[m * 16 + 4 * kq + 3]};
+    const u32x4 hv = ld128(s_h + m * TW + 8 * kq);
     const bf16x8_v av2 = act_frag(hv);
     const f32x4 tx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
         av2, as_frag(kOnes, kOnes, kOnes, kOnes), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -505,29 +531,31 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
   // D[i][j] of a 16x16 tile: lane j + 16*(i/4), element i%4 -> row 4*(lane>>4)+el; N-subtile t
   // of projection p holds column cl + t.
 #pragma unroll
-  for (int el = 0; el < 4; ++el) {
-    const int f = f_out[el];
+  for (int i = 0; i < EPW; ++i) {
+    const int f = f_out[i];
     if ((unsigned)f >= (unsigned)sd.num_slots) continue;
+    const int64_t o = (int64_t)f * NOUT + cl + j0;
     if constexpr (MODE == DEC_W1) {
-      uint32_t hp[CT / 2];
+      float hv[JPW];
 #pragma unroll
-      for (int j = 0; j < CT; j += 2)
-        hp[j / 2] = pack_bf16x2(silu_f32(acc[j][el]) * acc[CT + j][el],
-                                silu_f32(acc[j + 1][el]) * acc[CT + j + 1][el]);
-      uint16_t* dst = h_out + (int64_t)f * NOUT + cl;
-      if constexpr (CT == 2) {
-        *reinterpret_cast<uint32_t*>(dst) = hp[0];
+      for (int j = 0; j < JPW; ++j) hv[j] = silu_f32(fin[0][i][j]) * fin[1][i][j];
+      if constexpr (JPW == 1) {
+        h_out[o] = (uint16_t)f32_to_bf16_rne(hv[0]);
+      } else if constexpr (JPW == 2) {
+        *reinterpret_cast<uint32_t*>(h_out + o) = pack_bf16x2(hv[0], hv[1]);
       } else {
-        *reinterpret_cast<u32x2*>(dst) = u32x2{hp[0], hp[1]};
+        *reinterpret_cast<u32x2*>(h_out + o) =
+            u32x2{pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3])};
       }
     } else {
-      const float w = topk_w[f];
-      float* dst = ys + (int64_t)f * NOUT + cl;
-      if constexpr (CT == 2) {
-        *reinterpret_cast<float2*>(dst) = float2{w * acc[0][el], w * acc[1][el]};
+      const float w = w_out[i];
+      if constexpr (JPW == 1) {
+        ys[o] = w * fin[0][i][0];
+      } else if constexpr (JPW == 2) {
+        *reinterpret_cast<float2*>(ys + o) = float2{w * fin[0][i][0], w * fin[0][i][1]};
       } else {
-        *reinterpret_cast<float4*>(dst) =
-            float4{w * acc[0][el], w * acc[1][el], w * acc[2][el], w * acc[3][el]};
+        *reinterpret_cast<float4*>(ys + o) = float4{w * fin[0][i][0], w * fin[0][i][1],
+                                                    w * fin[0][i][2], w * fin[0][i][3]};
       }
     }
   }
@@ -554,6 +582,7 @@ __global__ __launch_bounds__(64 * kTokenSumMaxWaves) void w2_token_sum_kernel(
   const int G = ed.group, K = ed.inter, NOUT = ed.hidden;
   const int m = lane & 15, kq = lane >> 4;
   const int cl = blockIdx.x * TW + CT * m;
+  const float w = ok ? topk_w[f] : 0.0f;  // in flight with the weight stream
 
   f32x4 acc[CT];
 #pragma unroll
@@ -572,7 +601,6 @@ __global__ __launch_bounds__(64 * kTokenSumMaxWaves) void w2_token_sum_kernel(
       decode_tile<1, SPG, CT, NB>(tile, acc);
     }
   }
-  const float w = ok ? topk_w[f] : 0.0f;
   if (lane < 16) {  // row 0 of the tile: lanes 0..15, element 0
 #pragma unroll
     for (int j = 0; j < CT; ++j) part[i][CT * lane + j] = w * acc[j][0];
