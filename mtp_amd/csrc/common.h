@@ -75,17 +75,19 @@ MOE_DEV __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, uint32_t num_bytes) {
 // Resource over [base, base + 2 GiB) for data addressed by offsets below kOutOfRange.
 MOE_DEV __amdgpu_buffer_rsrc_t buf_rsrc(const void* base) { return buf_rsrc(base, kOutOfRange); }
 
+// soff: a further byte offset that is the same for the whole wave (a scalar register, so that the
+// loads of a loop share one lane offset).
 template <int AUX = 0>
-MOE_DEV u32x4 buf_ld128(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, AUX));
+MOE_DEV u32x4 buf_ld128(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff = 0) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, AUX));
 }
 template <int AUX = 0>
-MOE_DEV u32x2 buf_ld64(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, AUX));
+MOE_DEV u32x2 buf_ld64(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff = 0) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, AUX));
 }
 template <int AUX = 0>
-MOE_DEV uint32_t buf_ld32(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, AUX);
+MOE_DEV uint32_t buf_ld32(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff = 0) {
+  return __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, AUX);
 }
 
 // s_waitcnt immediate waiting for vmcnt <= n only (expcnt and lgkmcnt at their maximum).

@@ -103,7 +103,7 @@ struct AView {
 // cl .. cl + CT - 1. Every load is a buffer load from a uniform resource with a 32-bit lane
 // offset; group gi >= ngw (a ring stage past the slice) and padding rows load zeros with no
 // memory access, so the same instructions run on every path.
-template <int NP, int SPG, int CT>
+template <int NP, int SPG, int CT, int NGW = 0>  // NGW > 0: a slice of exactly NGW groups
 struct DecodeTile {
   __amdgpu_buffer_rsrc_t qr[NP], sr[NP], zr[NP];
   AView a;
@@ -113,7 +113,7 @@ struct DecodeTile {
 
   MOE_DEV DecodeTile(const ProjDev (&pj)[NP], AView av, int NOUT, int G_, int k0, int klen,
                      int cl, int kq)
-      : a(av), G(G_), ngw(klen / G_), zshift(4 * (cl & 7)) {
+      : a(av), G(G_), ngw(NGW > 0 ? NGW : klen / G_), zshift(4 * (cl & 7)) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       qr[p] = buf_rsrc(pj[p].qweight);
@@ -129,22 +129,27 @@ struct DecodeTile {
     zgrp = (uint32_t)(NOUT / 8) * 4u;
   }
 
+  // A lane's offsets stay the same for the whole slice; what moves from group to group and from
+  // k-step to k-step is uniform and goes into the loads' scalar offset (with the scales in the ring
+  // and one projection's group sums at a time: 190 -> 178 VGPRs in W1 with four columns per lane;
+  // eight layers of 64 tokens 509.6 -> 506.6 us, one layer of 203 95.2 -> 94.6 us).
   MOE_DEV void load_aw(GroupAW<NP, SPG, CT>& B, int gi) const {
     const uint32_t oob = gi < ngw ? 0u : kOutOfRange;
     const uint32_t ug = (uint32_t)gi;
 #pragma unroll
-    for (int s = 0; s < SPG; ++s) B.a[s] = buf_ld128(a.r, (a.off + (ug * G + 32 * s) * 2u) | oob);
+    for (int s = 0; s < SPG; ++s)
+      B.a[s] = buf_ld128(a.r, (a.off + (uint32_t)(64 * s)) | oob, ug * (uint32_t)G * 2u);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
 #pragma unroll
       for (int s = 0; s < SPG; ++s) {  // weights are streamed once: nontemporal
-        const uint32_t o = (qoff + ug * qgrp + (uint32_t)(4 * s) * qrow) | oob;
+        const uint32_t so = ug * qgrp + (uint32_t)(4 * s) * qrow;
         if constexpr (CT == 2) {
-          const u32x2 v = buf_ld64<kBufNontemporal>(qr[p], o);
+          const u32x2 v = buf_ld64<kBufNontemporal>(qr[p], qoff | oob, so);
           B.w[p][s][0] = v[0];
           B.w[p][s][1] = v[1];
         } else {
-          const u32x4 v = buf_ld128<kBufNontemporal>(qr[p], o);
+          const u32x4 v = buf_ld128<kBufNontemporal>(qr[p], qoff | oob, so);
 #pragma unroll
           for (int j = 0; j < 4; ++j) B.w[p][s][j] = v[j];
         }
@@ -158,13 +163,13 @@ struct DecodeTile {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       if constexpr (CT == 2) {
-        B.s[p][0] = buf_ld32(sr[p], (soff + ug * sgrp) | oob);
+        B.s[p][0] = buf_ld32(sr[p], soff | oob, ug * sgrp);
       } else {
-        const u32x2 v = buf_ld64(sr[p], (soff + ug * sgrp) | oob);
+        const u32x2 v = buf_ld64(sr[p], soff | oob, ug * sgrp);
         B.s[p][0] = v[0];
         B.s[p][1] = v[1];
       }
-      B.z[p] = buf_ld32(zr[p], (zoff + ug * zgrp) | oob);  // shifted at use: no wait here
+      B.z[p] = buf_ld32(zr[p], zoff | oob, ug * zgrp);  // shifted at use: no wait here
     }
   }
 
@@ -180,24 +185,27 @@ struct DecodeTile {
   }
   MOE_DEV void compute(const GroupAW<NP, SPG, CT>& B, const GroupSZ<NP, CT>& Z,
                        f32x4 (&acc)[NP * CT]) const {
-    constexpr int NT = NP * CT;
     const bf16x8_v ones = as_frag(kOnes, kOnes, kOnes, kOnes);
-    f32x4 tmp[NT], tx = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < NT; ++t) tmp[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 tx = {0.f, 0.f, 0.f, 0.f};
+    bf16x8_v av[SPG];
 #pragma unroll
     for (int s = 0; s < SPG; ++s) {
-      const bf16x8_v av = act_frag(B.a[s]);
-      tx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, ones, tx, 0, 0, 0);
+      av[s] = act_frag(B.a[s]);
+      tx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[s], ones, tx, 0, 0, 0);
+    }
+    // one projection after the other: the group sums of one are held at a time
 #pragma unroll
-      for (int p = 0; p < NP; ++p)
+    for (int p = 0; p < NP; ++p) {
+      f32x4 tmp[CT];
+#pragma unroll
+      for (int j = 0; j < CT; ++j) tmp[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < SPG; ++s) {
 #pragma unroll
         for (int j = 0; j < CT; ++j)
-          tmp[p * CT + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, weight_frag(B.w[p][s][j]),
-                                                                    tmp[p * CT + j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
+          tmp[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[s], weight_frag(B.w[p][s][j]),
+                                                           tmp[j], 0, 0, 0);
+      }
 #pragma unroll
       for (int j = 0; j < CT; ++j) {
         const uint32_t s2 = Z.s[p][j >> 1];
@@ -206,8 +214,9 @@ struct DecodeTile {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           acc[p * CT + j][i] =
-              __builtin_fmaf(sc, __builtin_fmaf(-zb, tx[i], tmp[p * CT + j][i]), acc[p * CT + j][i]);
+              __builtin_fmaf(sc, __builtin_fmaf(-zb, tx[i], tmp[j][i]), acc[p * CT + j][i]);
       }
+    }
   }
 };
 
@@ -241,26 +250,28 @@ MOE_DEV void static_for(F&& f) {
   }
 }
 
-// decode_tile for a K slice of exactly NGW groups as straight-line code: every group's scales
-// and zeros are loaded first, then a ring of DEPTH activation/weight buffers (DEPTH == NGW: all
-// loads up front). Without a loop back-edge each wait is for exactly the group about to be
+// decode_tile for a K slice of exactly NGW groups as straight-line code with a ring of DEPTH
+// buffers (DEPTH == NGW: all loads up front). Without a loop back-edge each wait is for exactly the group about to be
 // multiplied, whatever the ring depth.
 template <int NP, int SPG, int CT, int NGW, int DEPTH>
-MOE_DEV void decode_tile_static(const DecodeTile<NP, SPG, CT>& tile, f32x4 (&acc)[NP * CT]) {
+MOE_DEV void decode_tile_static(const DecodeTile<NP, SPG, CT, NGW>& tile, f32x4 (&acc)[NP * CT]) {
   static_assert(DEPTH >= 1 && DEPTH <= NGW, "ring depth within the slice");
-  GroupSZ<NP, CT> sz[NGW];
-  static_for<0, NGW>([&](auto gc) { tile.load_sz(sz[gc.value], gc.value); });
+  GroupSZ<NP, CT> sz[DEPTH];
   GroupAW<NP, SPG, CT> ring[DEPTH];
-  static_for<0, DEPTH - 1>([&](auto gc) { tile.load_aw(ring[gc.value], gc.value); });
+  static_for<0, DEPTH - 1>([&](auto gc) {
+    tile.load_sz(sz[gc.value], gc.value);
+    tile.load_aw(ring[gc.value], gc.value);
+  });
   static_for<0, NGW>([&](auto gc) {
     constexpr int g = gc.value;
     if constexpr (g + DEPTH - 1 < NGW) {
       __builtin_amdgcn_s_setprio(2);  // issue the stage's loads ahead of the other waves' math
+      tile.load_sz(sz[(g + DEPTH - 1) % DEPTH], g + DEPTH - 1);
       tile.load_aw(ring[(g + DEPTH - 1) % DEPTH], g + DEPTH - 1);
       __builtin_amdgcn_s_setprio(0);
     }
     __builtin_amdgcn_sched_barrier(0);  // this stage's loads before the wait for group g
-    tile.compute(ring[g % DEPTH], sz[g], acc);
+    tile.compute(ring[g % DEPTH], sz[g % DEPTH], acc);
   });
 }
 
@@ -394,7 +405,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
   const AView av{buf_rsrc(act, a_rows * (uint32_t)K * 2u),
                  valid_m ? (arow * (uint32_t)K + (uint32_t)(kw0 + 8 * kq)) * 2u : kOutOfRange};
   const int cl = blockIdx.x * TW + CT * m;  // this lane's first column
-  const DecodeTile<NP, SPG, CT> tile(pj, av, NOUT, G, kw0, kslice, cl, kq);
+  const DecodeTile<NP, SPG, CT, NB < 0 ? -NB : NGW> tile(pj, av, NOUT, G, kw0, kslice, cl, kq);
 
   // FW2: the down projection's words, scales and zeros for this wave's output columns, loaded
   // with the W1 stream. Lane (c = lane & 15, kq) takes packed row x * 4 + kq (TW == 32) and the
@@ -594,7 +605,7 @@ __global__ __launch_bounds__(64 * kTokenSumMaxWaves) void w2_token_sum_kernel(
     pj[0] = proj_row(pj[0], is_shared ? 0 : ed.row_stride, row, K / 8, K / G, NOUT);
     const AView av{buf_rsrc(h, (uint32_t)sd.num_slots * (uint32_t)K * 2u),
                    m == 0 ? ((uint32_t)f * (uint32_t)K + (uint32_t)(8 * kq)) * 2u : kOutOfRange};
-    const DecodeTile<1, SPG, CT> tile(pj, av, NOUT, G, 0, K, cl, kq);
+    const DecodeTile<1, SPG, CT, NB < 0 ? -NB : 0> tile(pj, av, NOUT, G, 0, K, cl, kq);
     if constexpr (NB < 0) {  // K is exactly -NB groups: every load up front
       decode_tile_static<1, SPG, CT, -NB, -NB>(tile, acc);
     } else {
