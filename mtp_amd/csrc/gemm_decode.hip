@@ -30,6 +30,8 @@
 // Arithmetic references: src/mtp_expert_prefetch/tracing/vllm_wna16_group_plan.py:367-486,
 // src/mtp_expert_prefetch/repack/gptq_unpack.py:88-131, 247-256, and the moe_sum order of
 // src/mtp_expert_prefetch/tracing/vllm_router_trace.py:19801-19804.
+#include <math.h>
+
 #include <type_traits>
 
 #include "common.h"
@@ -101,19 +103,19 @@ struct AView {
 
 // One wave's view of a K slice [k0, k0 + NGW*G) of the NP projections at columns
 // cl .. cl + CT - 1. Every load is a buffer load from a uniform resource with a 32-bit lane
-// offset; group gi >= ngw (a ring stage past the slice) and padding rows load zeros with no
-// memory access, so the same instructions run on every path.
-template <int NP, int SPG, int CT, int NGW = 0>  // NGW > 0: a slice of exactly NGW groups
+// offset; padding rows load zeros with no memory access, so the same instructions run on every
+// path.
+template <int NP, int SPG, int CT>
 struct DecodeTile {
   __amdgpu_buffer_rsrc_t qr[NP], sr[NP], zr[NP];
   AView a;
   uint32_t qoff, soff, zoff;        // lane offsets of group 0
   uint32_t qgrp, sgrp, zgrp, qrow;  // bytes per group (qweight, scales, zeros), per packed row
-  int G, ngw, zshift;
+  int G, zshift;
 
-  MOE_DEV DecodeTile(const ProjDev (&pj)[NP], AView av, int NOUT, int G_, int k0, int klen,
-                     int cl, int kq)
-      : a(av), G(G_), ngw(NGW > 0 ? NGW : klen / G_), zshift(4 * (cl & 7)) {
+  MOE_DEV DecodeTile(const ProjDev (&pj)[NP], AView av, int NOUT, int G_, int k0, int cl,
+                     int kq)
+      : a(av), G(G_), zshift(4 * (cl & 7)) {
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       qr[p] = buf_rsrc(pj[p].qweight);
@@ -134,22 +136,21 @@ struct DecodeTile {
   // and one projection's group sums at a time: 190 -> 178 VGPRs in W1 with four columns per lane;
   // eight layers of 64 tokens 509.6 -> 506.6 us, one layer of 203 95.2 -> 94.6 us).
   MOE_DEV void load_aw(GroupAW<NP, SPG, CT>& B, int gi) const {
-    const uint32_t oob = gi < ngw ? 0u : kOutOfRange;
     const uint32_t ug = (uint32_t)gi;
 #pragma unroll
     for (int s = 0; s < SPG; ++s)
-      B.a[s] = buf_ld128(a.r, (a.off + (uint32_t)(64 * s)) | oob, ug * (uint32_t)G * 2u);
+      B.a[s] = buf_ld128(a.r, a.off + (uint32_t)(64 * s), ug * (uint32_t)G * 2u);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
 #pragma unroll
       for (int s = 0; s < SPG; ++s) {  // weights are streamed once: nontemporal
         const uint32_t so = ug * qgrp + (uint32_t)(4 * s) * qrow;
         if constexpr (CT == 2) {
-          const u32x2 v = buf_ld64<kBufNontemporal>(qr[p], qoff | oob, so);
+          const u32x2 v = buf_ld64<kBufNontemporal>(qr[p], qoff, so);
           B.w[p][s][0] = v[0];
           B.w[p][s][1] = v[1];
         } else {
-          const u32x4 v = buf_ld128<kBufNontemporal>(qr[p], qoff | oob, so);
+          const u32x4 v = buf_ld128<kBufNontemporal>(qr[p], qoff, so);
 #pragma unroll
           for (int j = 0; j < 4; ++j) B.w[p][s][j] = v[j];
         }
@@ -158,18 +159,17 @@ struct DecodeTile {
   }
 
   MOE_DEV void load_sz(GroupSZ<NP, CT>& B, int gi) const {
-    const uint32_t oob = gi < ngw ? 0u : kOutOfRange;
     const uint32_t ug = (uint32_t)gi;
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       if constexpr (CT == 2) {
-        B.s[p][0] = buf_ld32(sr[p], soff | oob, ug * sgrp);
+        B.s[p][0] = buf_ld32(sr[p], soff, ug * sgrp);
       } else {
-        const u32x2 v = buf_ld64(sr[p], soff | oob, ug * sgrp);
+        const u32x2 v = buf_ld64(sr[p], soff, ug * sgrp);
         B.s[p][0] = v[0];
         B.s[p][1] = v[1];
       }
-      B.z[p] = buf_ld32(zr[p], zoff | oob, ug * zgrp);  // shifted at use: no wait here
+      B.z[p] = buf_ld32(zr[p], zoff, ug * zgrp);  // shifted at use: no wait here
     }
   }
 
@@ -220,27 +220,6 @@ struct DecodeTile {
   }
 };
 
-// One wave: acc[p*CT + j] += A[16 rows, k0 : k0+klen] . W_p[k0 : k0+klen, cl + j] for the NP
-// projections, klen a multiple of G. A ring of NB group buffers keeps groups g + 1 .. g + NB - 1
-// in flight while group g is multiplied; the loop body issues the same loads on every pass
-// (stages past the slice read zeros), so each wait is for exactly the group about to be used.
-template <int NP, int SPG, int CT, int NB>
-MOE_DEV void decode_tile(const DecodeTile<NP, SPG, CT>& tile, f32x4 (&acc)[NP * CT]) {
-  GroupBuf<NP, SPG, CT> ring[NB];
-#pragma unroll
-  for (int j = 0; j < NB - 1; ++j) tile.load(ring[j], j);
-  for (int g0 = 0; g0 < tile.ngw; g0 += NB) {
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      tile.load(ring[(j + NB - 1) % NB], g0 + j + NB - 1);
-      // keep the stage's loads ahead of the wait for group g0 + j (the scheduler would sink
-      // them below it, leaving one group in flight)
-      __builtin_amdgcn_sched_barrier(0);
-      tile.compute(ring[j], acc);
-    }
-  }
-}
-
 // Compile-time loop: f(std::integral_constant<int, I>) for I in [B, E).
 template <int B, int E, typename F>
 MOE_DEV void static_for(F&& f) {
@@ -250,11 +229,13 @@ MOE_DEV void static_for(F&& f) {
   }
 }
 
-// decode_tile for a K slice of exactly NGW groups as straight-line code with a ring of DEPTH
-// buffers (DEPTH == NGW: all loads up front). Without a loop back-edge each wait is for exactly the group about to be
+// One wave: acc[p*CT + j] += A[16 rows, k0 : k0+klen] . W_p[k0 : k0+klen, cl + j] for the NP
+// projections over a slice of exactly NGW groups, as straight-line code with a ring of DEPTH
+// buffers (DEPTH == NGW: all loads up front): groups g + 1 .. g + DEPTH - 1 are in flight while
+// group g is multiplied. Without a loop back-edge each wait is for exactly the group about to be
 // multiplied, whatever the ring depth.
 template <int NP, int SPG, int CT, int NGW, int DEPTH>
-MOE_DEV void decode_tile_static(const DecodeTile<NP, SPG, CT, NGW>& tile, f32x4 (&acc)[NP * CT]) {
+MOE_DEV void decode_tile(const DecodeTile<NP, SPG, CT>& tile, f32x4 (&acc)[NP * CT]) {
   static_assert(DEPTH >= 1 && DEPTH <= NGW, "ring depth within the slice");
   GroupSZ<NP, CT> sz[DEPTH];
   GroupAW<NP, SPG, CT> ring[DEPTH];
@@ -290,15 +271,13 @@ MOE_DEV void projections(const ExpertsDev& ed, int mode, bool is_shared, ProjDev
 // alone doing it, the sums, SiLUs and stores of the whole tile were a serial tail of each
 // workgroup (eight layers: of one token 160 -> 156 us, of 64 518 -> 508 us; of 48 with 64 experts
 // 159 -> 153 us; one layer of 203 tokens 97.4 -> 95.5 us).
-// NB > 0 and NGW == 0: runtime loop over the wave's groups with an NB-deep ring; NB < 0: a
-// slice of exactly -NB groups, all loaded up front; NGW > 0: a slice of exactly NGW groups with
-// an NB-deep ring, unrolled.
+// A wave's slice has exactly NGW groups, loaded through an NB-deep ring (NB == NGW: all up front).
 // FW2 (W1 on the slot grid, CT == 2): W2 fused in. The block's 32 h columns are the K rows
 // [32 x, 32 x + 32) of the down projection (inside one quantisation group); after the W1
 // epilogue every wave multiplies the block's h rows (from LDS) by its kW2Groups x 64 output
 // columns and writes the weighted fp32 partial rows ys[slot][x][n] (partial_sum adds them).
 // The workgroup of a dropped expert writes zero rows, so every partial row is written.
-template <int MODE, int SPG, int KS, int CT, int NB, int NGW = 0, bool FW2 = false>
+template <int MODE, int SPG, int KS, int CT, int NB, int NGW, bool FW2 = false>
 __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
     const uint16_t* __restrict__ act, ExpertsDev ed, SlotsDev sd,
     const int32_t* __restrict__ sorted, const int32_t* __restrict__ eids,
@@ -405,7 +384,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
   const AView av{buf_rsrc(act, a_rows * (uint32_t)K * 2u),
                  valid_m ? (arow * (uint32_t)K + (uint32_t)(kw0 + 8 * kq)) * 2u : kOutOfRange};
   const int cl = blockIdx.x * TW + CT * m;  // this lane's first column
-  const DecodeTile<NP, SPG, CT, NB < 0 ? -NB : NGW> tile(pj, av, NOUT, G, kw0, kslice, cl, kq);
+  const DecodeTile<NP, SPG, CT> tile(pj, av, NOUT, G, kw0, cl, kq);
 
   // FW2: the down projection's words, scales and zeros for this wave's output columns, loaded
   // with the W1 stream. Lane (c = lane & 15, kq) takes packed row x * 4 + kq (TW == 32) and the
@@ -446,15 +425,9 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
   f32x4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if constexpr (NB < 0) {  // fixed: the wave's slice is exactly -NB groups, all loads up front
-    decode_tile_static<NP, SPG, CT, -NB, -NB>(tile, acc);
-  } else if constexpr (NGW > 0) {
-    decode_tile_static<NP, SPG, CT, NGW, NB>(tile, acc);
-  } else {
-    decode_tile<NP, SPG, CT, NB>(tile, acc);
-  }
+  decode_tile<NP, SPG, CT, NGW, NB>(tile, acc);
 
-  // This wave's share: out[p][i][j] = element el0 + i of N-subtile j0 + j of projection p, the
+  // This wave's share: fin[p][i][j] = element el0 + i of N-subtile j0 + j of projection p, the
   // waves' partial sums added in wave order.
   float fin[NP][EPW][JPW];
   if constexpr (KS > 1) {
@@ -575,7 +548,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_decode_kernel(
 // Token-major W2 + weighted sum: block (column tile, token t); wave i < top_k handles routed slot
 // t*top_k + i, wave top_k (when present) the shared slot T*top_k + t. A = h[slot] in MFMA row 0
 // (the other 15 rows are zero); the block adds the waves' w[slot] * y rows in slot order.
-template <int SPG, int CT, int NB>
+template <int SPG, int CT, int NGW, int NB>
 __global__ __launch_bounds__(64 * kTokenSumMaxWaves) void w2_token_sum_kernel(
     const uint16_t* __restrict__ h, ExpertsDev ed, SlotsDev sd, const int32_t* __restrict__ ids,
     const float* __restrict__ topk_w, uint16_t* __restrict__ out) {
@@ -605,12 +578,8 @@ __global__ __launch_bounds__(64 * kTokenSumMaxWaves) void w2_token_sum_kernel(
     pj[0] = proj_row(pj[0], is_shared ? 0 : ed.row_stride, row, K / 8, K / G, NOUT);
     const AView av{buf_rsrc(h, (uint32_t)sd.num_slots * (uint32_t)K * 2u),
                    m == 0 ? ((uint32_t)f * (uint32_t)K + (uint32_t)(8 * kq)) * 2u : kOutOfRange};
-    const DecodeTile<1, SPG, CT, NB < 0 ? -NB : 0> tile(pj, av, NOUT, G, 0, K, cl, kq);
-    if constexpr (NB < 0) {  // K is exactly -NB groups: every load up front
-      decode_tile_static<1, SPG, CT, -NB, -NB>(tile, acc);
-    } else {
-      decode_tile<1, SPG, CT, NB>(tile, acc);
-    }
+    const DecodeTile<1, SPG, CT> tile(pj, av, NOUT, G, 0, cl, kq);
+    decode_tile<1, SPG, CT, NGW, NB>(tile, acc);
   }
   if (lane < 16) {  // row 0 of the tile: lanes 0..15, element 0
 #pragma unroll
@@ -633,7 +602,7 @@ bool decode_offsets_fit(const ExpertsDev& ed, const SlotsDev& sd) {
          (int64_t)ed.hidden * ed.inter / 2 < lim;
 }
 
-template <int MODE, int SPG, int KS, int CT, int NB, int NGW = 0>
+template <int MODE, int SPG, int KS, int CT, int NB, int NGW>
 hipError_t launch_cfg(const uint16_t* act, const ExpertsDev& ed, const SlotsDev& sd,
                       const int32_t* sorted, const int32_t* eids, const int32_t* ntpp, int cap,
                       const float* topk_w, uint16_t* h, float* ys, const SlotGrid& sg,
@@ -646,110 +615,83 @@ hipError_t launch_cfg(const uint16_t* act, const ExpertsDev& ed, const SlotsDev&
   return hipGetLastError();
 }
 
-template <int MODE, int KS, int CT, int NB>
-hipError_t launch_group(const uint16_t* act, const ExpertsDev& ed, const SlotsDev& sd,
-                        const int32_t* sorted, const int32_t* eids, const int32_t* ntpp, int cap,
-                        const float* topk_w, uint16_t* h, float* ys, const SlotGrid& sg,
-                        hipStream_t stream) {
-  switch (ed.group) {
-    case 64: return launch_cfg<MODE, 2, KS, CT, NB>(act, ed, sd, sorted, eids, ntpp, cap, topk_w, h, ys, sg, stream);
-    case 128: return launch_cfg<MODE, 4, KS, CT, NB>(act, ed, sd, sorted, eids, ntpp, cap, topk_w, h, ys, sg, stream);
-    case 256: return launch_cfg<MODE, 8, KS, CT, NB>(act, ed, sd, sorted, eids, ntpp, cap, topk_w, h, ys, sg, stream);
-    default: return hipErrorInvalidValue;
-  }
-}
+// Tile of a decode GEMM: ks waves over K, 16 * ct columns.
+struct DecodeCfg {
+  int ks, ct;
+};
 
-// Any valid (waves per block, columns per lane, ring depth[, groups per wave]) configuration.
-// ngw > 0 selects the unrolled ring over exactly ngw groups per wave (group size 128 only).
-template <int MODE>
+// Every configuration that pick_decode_cfg gives for hidden in {512, 1024, 1536, 2048},
+// intermediate in {256, 512, 1024} and groups of 32 SPG.
+template <int MODE, int SPG>
 hipError_t launch_decode_cfg(const uint16_t* act, const ExpertsDev& ed, const SlotsDev& sd,
                              const int32_t* sorted, const int32_t* eids, const int32_t* ntpp,
-                             int cap, const float* topk_w, uint16_t* h, float* ys, int ks, int ct,
-                             int nb, int ngw, const SlotGrid& sg, hipStream_t stream) {
+                             int cap, const float* topk_w, uint16_t* h, float* ys, DecodeCfg c,
+                             const SlotGrid& sg, hipStream_t stream) {
   const int K = (MODE == DEC_W1) ? ed.hidden : ed.inter;
   const int NOUT = (MODE == DEC_W1) ? ed.inter : ed.hidden;
-  if ((ct != 2 && ct != 4) || NOUT % (16 * ct) != 0 || K % (ks * ed.group) != 0)
-    return hipErrorInvalidValue;
-  if (nb < 0 && K / (ks * ed.group) != -nb) return hipErrorInvalidValue;
-  if (ngw > 0) {
-    if (ed.group != 128 || K / (ks * ed.group) != ngw || nb < 1 || nb > ngw)
-      return hipErrorInvalidValue;
-#define MOE_DEC_STATIC(KSV, CTV, NBV, NGWV)                                                     \
-    if (ks == KSV && ct == CTV && nb == NBV && ngw == NGWV)                                     \
-      return launch_cfg<MODE, 4, KSV, CTV, NBV, NGWV>(act, ed, sd, sorted, eids, ntpp, cap,     \
-                                                      topk_w, h, ys, sg, stream);
-    MOE_DEC_STATIC(4, 4, 2, 4) MOE_DEC_STATIC(4, 4, 3, 4) MOE_DEC_STATIC(4, 2, 2, 4)
-    MOE_DEC_STATIC(4, 2, 3, 4) MOE_DEC_STATIC(2, 2, 2, 8) MOE_DEC_STATIC(2, 2, 3, 8)
-    MOE_DEC_STATIC(2, 4, 2, 8) MOE_DEC_STATIC(2, 4, 3, 8) MOE_DEC_STATIC(1, 4, 2, 4)
-    MOE_DEC_STATIC(1, 4, 3, 4) MOE_DEC_STATIC(1, 2, 2, 4) MOE_DEC_STATIC(1, 2, 3, 4)
-#undef MOE_DEC_STATIC
-    return hipErrorInvalidValue;
+  if (NOUT % (16 * c.ct) != 0 || K % (c.ks * ed.group) != 0) return hipErrorInvalidValue;
+  const int ngw = K / (c.ks * ed.group);
+#define MOE_DEC(KSV, CTV, NGWV)                                                                \
+  if (c.ks == KSV && c.ct == CTV && ngw == NGWV)                                               \
+    return launch_cfg<MODE, SPG, KSV, CTV, (NGWV < 2 ? NGWV : 2), NGWV>(                       \
+        act, ed, sd, sorted, eids, ntpp, cap, topk_w, h, ys, sg, stream);
+#define MOE_DEC2(KSV, NGWV) MOE_DEC(KSV, 2, NGWV) MOE_DEC(KSV, 4, NGWV)
+  if constexpr (MODE == DEC_W1) {
+    if constexpr (SPG == 2) { MOE_DEC2(4, 2) MOE_DEC2(4, 4) MOE_DEC2(4, 6) MOE_DEC2(4, 8) }
+    if constexpr (SPG == 4) { MOE_DEC2(4, 1) MOE_DEC2(4, 2) MOE_DEC2(4, 3) MOE_DEC2(4, 4) }
+    if constexpr (SPG == 8) { MOE_DEC2(4, 1) MOE_DEC2(4, 2) MOE_DEC2(2, 1) MOE_DEC2(2, 3) }
+    MOE_DEC(8, 2, 1)
+    if constexpr (SPG <= 4) { MOE_DEC(8, 2, 2) }
+    if constexpr (SPG == 2) { MOE_DEC(8, 2, 3) MOE_DEC(8, 2, 4) }
+  } else {
+    MOE_DEC(4, 4, 1)
+    if constexpr (SPG <= 4) { MOE_DEC(4, 4, 2) }
+    if constexpr (SPG == 2) { MOE_DEC(4, 4, 4) }
+    if constexpr (SPG >= 4) { MOE_DEC(2, 4, 1) }
+    if constexpr (SPG == 8) { MOE_DEC(1, 4, 1) }
   }
-#define MOE_DEC_CASE(KSV, CTV, NBV)                                                             \
-  if (ks == KSV && ct == CTV && nb == NBV)                                                      \
-    return launch_group<MODE, KSV, CTV, NBV>(act, ed, sd, sorted, eids, ntpp, cap, topk_w, h,  \
-                                             ys, sg, stream);
-  MOE_DEC_CASE(1, 2, 2) MOE_DEC_CASE(2, 2, 2) MOE_DEC_CASE(4, 2, 2) MOE_DEC_CASE(8, 2, 2)
-  MOE_DEC_CASE(1, 4, 2) MOE_DEC_CASE(2, 4, 2) MOE_DEC_CASE(4, 4, 2)
-  // fixed slices (nb = -groups per wave), all loads in flight at once
-  MOE_DEC_CASE(1, 2, -4) MOE_DEC_CASE(2, 2, -4) MOE_DEC_CASE(4, 2, -4) MOE_DEC_CASE(8, 2, -2)
-  MOE_DEC_CASE(1, 4, -4) MOE_DEC_CASE(2, 4, -4) MOE_DEC_CASE(4, 4, -4) MOE_DEC_CASE(8, 4, -2)
-  MOE_DEC_CASE(2, 2, -2) MOE_DEC_CASE(4, 2, -2) MOE_DEC_CASE(2, 4, -2) MOE_DEC_CASE(4, 4, -2)
-  MOE_DEC_CASE(1, 2, -2) MOE_DEC_CASE(1, 4, -2)
-#undef MOE_DEC_CASE
+#undef MOE_DEC2
+#undef MOE_DEC
   return hipErrorInvalidValue;
 }
 
-// Configuration by problem size (measured on MI355X, 40 Zipf-skewed layers of H 2048, I 512,
-// E 256, top-8, group 128; num_slots 8 / 64 / 256 / 512 at batch 1 / 8 / 32 / 64):
-//   W1: up to 16 slots, 8 waves over K with both of a wave's groups loaded up front (7.2 us);
-//       up to 384 slots, four waves over K, two columns per lane, unrolled 2-deep ring over the
-//       wave's 4 groups (13.6 us at 64 slots, 23.0 us at 256); beyond, the same with four
-//       columns per lane (31.3 us at 512).
-//   W2 (K = 512, four columns per lane): two waves over K with both groups up front (7.9 us at
-//       64 slots, 17.1 us at 512), except between 128 and 384 slots where one wave with an
-//       unrolled 2-deep ring over its 4 groups is faster (12.6 vs 13.1 us).
-// The unrolled rings exist for group size 128 and the slices above; other shapes use the
-// runtime ring with the same waves and columns.
+// Configuration by problem size, from sweeps over hidden 512 .. 2048, intermediate 256 .. 1024,
+// groups of 64 .. 256 and 4 .. 203 tokens (times of eight layers, 128 or 256 experts):
+//  - Four waves over K wherever the groups divide by four: now that all of a block's waves finish
+//    its tile, more waves cost no longer tail (W2 of 64 tokens, K 512: four waves of one group
+//    491.7 us, two of two 497.5, one of four 505).
+//  - A wave's groups unrolled with a 2-deep ring: all other forms are slower, a runtime loop by
+//    most (W1 of 32 tokens 393 against 446 us; W1 with K 2048 in groups of 256, 48 tokens, 636
+//    against 773); deeper rings and more waves per SIMD too.
+//  - W1 with four columns per lane (half the activation loads per weight) from about 700
+//    workgroups of that size on (32 tokens: 393 against 409 us with two), and where they are
+//    about one for each of the 256 CUs (hidden 2048, 4 tokens: 192.5 against 205.8); between
+//    these some CUs would get one such workgroup and others two (8 tokens: 267 against 257), and
+//    below there are too few. The workgroups are estimated from the experts that an even routing
+//    reaches. K of 512 is too short to gain from it (64 tokens: 239 against 234 us).
+//  - Up to 16 slots W1 takes eight waves: nothing but latency counts there.
 template <int MODE>
-void pick_decode_cfg(const ExpertsDev& ed, const SlotsDev& sd, int* ks, int* ct, int* nb,
-                     int* ngw) {
-  *ngw = 0;
+DecodeCfg pick_decode_cfg(const ExpertsDev& ed, const SlotsDev& sd) {
   const int K = (MODE == DEC_W1) ? ed.hidden : ed.inter;
   const int groups = K / ed.group;
-  const int slots = sd.num_slots;
-  auto fixed = [&](int k) {  // k waves over K, all of a wave's groups in flight
-    if (k >= 1 && groups % k == 0 && (groups / k == 4 || groups / k == 2)) {
-      *ks = k;
-      *nb = -(groups / k);
-      return true;
-    }
-    return false;
-  };
-  auto ring = [&](int k, int unrolled_groups) {  // k waves over K, 2-deep ring
-    *ks = k;
-    *nb = 2;
-    while (*ks > 1 && K % (*ks * ed.group) != 0) *ks /= 2;
-    if (ed.group == 128 && *ks == k && K == k * 128 * unrolled_groups) *ngw = unrolled_groups;
-  };
+  DecodeCfg c{groups % 4 == 0 ? 4 : (groups % 2 == 0 ? 2 : 1), 4};
   if (MODE == DEC_W1) {
-    *ct = 2;
-    if (slots <= 16 && fixed(groups / 2)) return;
-    if (slots > 384 && ed.inter % 64 == 0) *ct = 4;
-    return ring(4, 4);
+    const float E = (float)ed.num_experts;
+    const float reached = E * (1.0f - powf(fmaxf(0.0f, 1.0f - (float)sd.top_k / E), (float)sd.T));
+    const float wgs = reached * (float)(ed.inter / 64);
+    if (K <= 512 || wgs < 220.0f || (wgs > 300.0f && wgs < 700.0f)) c.ct = 2;
+    if (sd.num_slots <= 16 && groups % 8 == 0) c = DecodeCfg{8, 2};
   }
-  *ct = ed.hidden % 64 == 0 ? 4 : 2;
-  if ((slots <= 128 || slots > 384) && fixed(groups / 2)) return;
-  ring(1, 4);
+  return c;
 }
 
-template <int SPG, int CT, int NB>
+template <int SPG, int CT, int NGW, int NB>
 hipError_t launch_token_sum(const uint16_t* h, const ExpertsDev& ed, const SlotsDev& sd,
                             const int32_t* ids, const float* topk_w, uint16_t* out,
                             hipStream_t stream) {
   const int has_shared = sd.num_slots > sd.T * sd.top_k ? 1 : 0;
   const dim3 grid(ed.hidden / (16 * CT), sd.T);
-  hipLaunchKernelGGL((w2_token_sum_kernel<SPG, CT, NB>), grid, dim3(64 * (sd.top_k + has_shared)),
+  hipLaunchKernelGGL((w2_token_sum_kernel<SPG, CT, NGW, NB>), grid, dim3(64 * (sd.top_k + has_shared)),
                      0, stream, h, ed, sd, ids, topk_w, out);
   return hipGetLastError();
 }
@@ -762,14 +704,17 @@ hipError_t launch_decode_picked(const uint16_t* act, const ExpertsDev& ed, const
                                 const int32_t* sorted, const int32_t* eids, const int32_t* ntpp,
                                 int cap, const float* topk_w, uint16_t* h, float* ys,
                                 const SlotGrid& sg, hipStream_t stream) {
-  int ks, ct, nb, ngw;
-  pick_decode_cfg<MODE>(ed, sd, &ks, &ct, &nb, &ngw);
-  hipError_t e = launch_decode_cfg<MODE>(act, ed, sd, sorted, eids, ntpp, cap, topk_w, h, ys, ks,
-                                         ct, nb, ngw, sg, stream);
-  if (e == hipErrorInvalidValue)  // shape outside the tuned set: one wave, double-buffered
-    e = launch_decode_cfg<MODE>(act, ed, sd, sorted, eids, ntpp, cap, topk_w, h, ys, 1, 2, 2, 0,
-                                sg, stream);
-  return e;
+  auto launch = [&](auto spg, DecodeCfg c) {
+    return launch_decode_cfg<MODE, decltype(spg)::value>(act, ed, sd, sorted, eids, ntpp, cap,
+                                                         topk_w, h, ys, c, sg, stream);
+  };
+  DecodeCfg c = pick_decode_cfg<MODE>(ed, sd);
+  switch (ed.group) {
+    case 64: return launch(std::integral_constant<int, 2>{}, c);
+    case 128: return launch(std::integral_constant<int, 4>{}, c);
+    case 256: return launch(std::integral_constant<int, 8>{}, c);
+    default: return hipErrorInvalidValue;
+  }
 }
 }  // namespace
 
@@ -821,7 +766,7 @@ hipError_t launch_w1w2_slotgrid(const uint16_t* x, const ExpertsDev& ed, const S
   switch (ed.hidden / 256) {
 #define MOE_W1W2(KSV)                                                                          \
   case KSV:                                                                                    \
-    hipLaunchKernelGGL((gemm_decode_kernel<DEC_W1, 4, KSV, 2, -2, 0, true>), grid,             \
+    hipLaunchKernelGGL((gemm_decode_kernel<DEC_W1, 4, KSV, 2, 2, 2, true>), grid,             \
                        dim3(64 * KSV), 0, stream, x, ed, sd, nullptr, nullptr, nullptr,        \
                        nullptr, nullptr, part, sg);                                            \
     return hipGetLastError();
@@ -841,17 +786,13 @@ hipError_t launch_w2_token_sum(const uint16_t* h, const ExpertsDev& ed, const Sl
                                const int32_t* ids, const float* topk_w, uint16_t* out,
                                hipStream_t stream) {
   if (!w2_token_sum_fits(ed, sd) || !decode_offsets_fit(ed, sd)) return hipErrorInvalidValue;
-  const int groups = ed.inter / ed.group;
-  switch (ed.group) {  // K = 512: all of a slot's groups in flight at once; else a 2-deep ring
-    case 64:
-      return groups == 8 ? launch_token_sum<2, 2, -8>(h, ed, sd, ids, topk_w, out, stream)
-                         : launch_token_sum<2, 2, 2>(h, ed, sd, ids, topk_w, out, stream);
-    case 128:
-      return groups == 4 ? launch_token_sum<4, 2, -4>(h, ed, sd, ids, topk_w, out, stream)
-                         : launch_token_sum<4, 2, 2>(h, ed, sd, ids, topk_w, out, stream);
-    case 256:
-      return groups == 2 ? launch_token_sum<8, 2, -2>(h, ed, sd, ids, topk_w, out, stream)
-                         : launch_token_sum<8, 2, 2>(h, ed, sd, ids, topk_w, out, stream);
-    default: return hipErrorInvalidValue;
-  }
+  // K of 256 and 512: all of a slot's groups in flight at once; K of 1024: 512 k of them.
+#define MOE_TOKEN_SUM(G, K, NGW, NB)     \
+  if (ed.group == G && ed.inter == K)    \
+    return launch_token_sum<G / 32, 2, NGW, NB>(h, ed, sd, ids, topk_w, out, stream);
+  MOE_TOKEN_SUM(64, 256, 4, 4) MOE_TOKEN_SUM(64, 512, 8, 8) MOE_TOKEN_SUM(64, 1024, 16, 8)
+  MOE_TOKEN_SUM(128, 256, 2, 2) MOE_TOKEN_SUM(128, 512, 4, 4) MOE_TOKEN_SUM(128, 1024, 8, 4)
+  MOE_TOKEN_SUM(256, 256, 1, 1) MOE_TOKEN_SUM(256, 512, 2, 2) MOE_TOKEN_SUM(256, 1024, 4, 2)
+#undef MOE_TOKEN_SUM
+  return hipErrorInvalidValue;
 }

@@ -94,6 +94,19 @@ def test_decode_shapes_and_groups(E, H, I, G, shared, T):
     _check_layer(layer, T, 4, "decode")
 
 
+@pytest.mark.parametrize("H", [512, 1024, 1536, 2048])
+@pytest.mark.parametrize("G", [64, 128, 256])
+def test_decode_tiles(H, G):
+    """Every tile of the decode GEMMs (waves over K, groups per wave, columns per lane): 12 tokens
+    take two columns per lane in W1 at intermediate 256 and 512 and, from hidden 1024 on, four at
+    1024 (about 250 workgroups); 2 tokens eight waves over K where the groups allow it, 5 the
+    token-sum W2 of each intermediate size."""
+    for I, T in ((256, 12), (512, 12), (1024, 12), (512, 2), (256, 5), (512, 5), (1024, 5)):
+        _say(f"decode tiles H={H} G={G} I={I} T={T}")
+        layer = synth.make_layer(4, num_experts=16, hidden=H, intermediate=I, group=G)
+        _check_layer(layer, T, 4, "decode")
+
+
 @pytest.mark.parametrize("T", [1, 32])
 def test_config4_shared_expert(T):
     """Config 4: routed top-8 plus a sigmoid-gated int4 shared expert."""
