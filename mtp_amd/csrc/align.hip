@@ -8,15 +8,15 @@
 // ballot-based match, which leaves its per-expert counts in LDS; the counts become exclusive
 // per-(wave, expert) base positions, and every slot goes to base + rank. The order is therefore
 // experts ascending, slots ascending within an expert - a stable argsort.
-// Large inputs (prefill): the same ranking per chunk in many single-wave workgroups, then one
-// block for the offsets and the scatter (align_chunk_kernel / align_finish_kernel below).
+// Large inputs (prefill): the same ranking per chunk in many small workgroups, then one block
+// for the offsets and the scatter (align_chunk_kernel / align_finish_kernel below).
 #include "launch.h"
 #include "routing.h"
 
 namespace {
 
 // ---- Two-kernel align for large inputs (prefill): chunk ranks in parallel, then one block.
-// Kernel 1: workgroup c (one wave) ranks the slots of chunk c = [c CH, (c + 1) CH) by expert in
+// Kernel 1: workgroup c ranks the slots of chunk c = [c CH, (c + 1) CH) by expert in
 // slot order (the ballot match of align_block, 64 slots at a time) and writes, into the sorted
 // buffer used as scratch, each slot's rank inside its chunk at sorted[f] and the chunk's
 // per-group counts at sorted[n_slots + c G + g].
@@ -29,39 +29,74 @@ constexpr int kAlign2MaxChunks = 64;
 constexpr int kAlign2LdsCounts = 16448;       // chunks x groups held in LDS by kernel 2
 constexpr int kAlign2MaxSlotsPerThread = 32;  // kernel 2's registers: slots of one thread
 
-__global__ __launch_bounds__(64) void align_chunk_kernel(const int32_t* __restrict__ topk_ids,
-                                                         int T, int top_k, int E, int has_shared,
-                                                         int CH, int32_t* __restrict__ scratch) {
-  __shared__ int cnt[kMaxGroups];
-  const int lane = threadIdx.x, c = blockIdx.x;
+// The chunk is dealt to kChunkWaves waves in slot order; their counts become bases inside the chunk
+// and the ranks are written once. A wave's chain over its slots, 64 at a time, is what bounds the
+// kernel: with one wave for the whole chunk a layer of 8192 tokens took 612.9 us, with four 610.0.
+constexpr int kChunkWaves = 4;
+__global__ __launch_bounds__(64 * kChunkWaves) void align_chunk_kernel(
+    const int32_t* __restrict__ topk_ids, int T, int top_k, int E, int has_shared, int CH,
+    int32_t* __restrict__ scratch) {
+  __shared__ int cnt[kChunkWaves][kMaxGroups];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = blockIdx.x;
   const int routed = T * top_k;
   const int n_slots = routed + (has_shared ? T : 0);
   const int G = E + (has_shared ? 1 : 0);
-  for (int g = lane; g < G; g += 64) cnt[g] = 0;
-  __builtin_amdgcn_wave_barrier();
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // one wave: LDS ops complete in order
-  const int lo = min(c * CH, n_slots), hi = min(lo + CH, n_slots);
+  const int per_wave = (CH + 64 * kChunkWaves - 1) / (64 * kChunkWaves) * 64;
+  const int end = min(c * CH + CH, n_slots);
+  const int lo = min(c * CH + w * per_wave, end), hi = min(lo + per_wave, end);
   const __amdgpu_buffer_rsrc_t ir = buf_rsrc(topk_ids, (uint32_t)routed * 4u);
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const bool held = per_wave <= 64 * kAlignIds;  // uniform over the workgroup
+  int eb[kAlignIds], rank[kAlignIds];
+  align_ids(ir, routed, E, lo, hi, lane, eb);
+  // every wave clears and fills its own counters: LDS operations of one wave complete in order
+  for (int g = lane; g < G; g += 64) cnt[w][g] = 0;
+  __builtin_amdgcn_wave_barrier();
+  // ranks inside the wave's range: held in registers, or written and read back (longer ranges)
   for (int base0 = lo; base0 < hi; base0 += 64 * kAlignIds) {
-    int eb[kAlignIds];
-    align_ids(ir, routed, E, base0, hi, lane, eb);
+    if (base0 > lo) align_ids(ir, routed, E, base0, hi, lane, eb);
 #pragma unroll
     for (int u = 0; u < kAlignIds; ++u) {
       const int f = base0 + 64 * u + lane;
-      if (base0 + 64 * u >= hi) break;  // uniform
+      if (base0 + 64 * u >= hi) break;  // uniform over the wave
       const int e = eb[u];
-      const bool valid = e >= 0;
       const uint64_t peers = expert_peers(e);
-      if (valid) scratch[f] = cnt[e] + __popcll(peers & lt_mask);
+      const int before = e >= 0 ? cnt[w][e] : 0;
+      rank[u] = before + __popcll(peers & lt_mask);
+      if (!held && e >= 0) scratch[f] = rank[u];
+      __builtin_amdgcn_wave_barrier();  // every lane has read the old count
+      if (e >= 0 && (peers & lt_mask) == 0) cnt[w][e] = before + __popcll(peers);
       __builtin_amdgcn_wave_barrier();
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (valid && (__ffsll((long long)peers) - 1) == lane) cnt[e] += __popcll(peers);
-      __builtin_amdgcn_wave_barrier();
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   }
-  for (int g = lane; g < G; g += 64) scratch[n_slots + c * G + g] = cnt[g];
+  __syncthreads();
+  for (int g = tid; g < G; g += 64 * kChunkWaves) {
+    int run = 0;
+#pragma unroll
+    for (int v = 0; v < kChunkWaves; ++v) {
+      const int n = cnt[v][g];
+      cnt[v][g] = run;
+      run += n;
+    }
+    scratch[n_slots + c * G + g] = run;
+  }
+  __syncthreads();
+  if (held) {
+#pragma unroll
+    for (int u = 0; u < kAlignIds; ++u) {
+      if (lo + 64 * u >= hi) break;  // uniform over the wave
+      if (eb[u] >= 0) scratch[lo + 64 * u + lane] = cnt[w][eb[u]] + rank[u];
+    }
+  } else {
+    for (int base0 = lo; base0 < hi; base0 += 64 * kAlignIds) {
+      align_ids(ir, routed, E, base0, hi, lane, eb);
+#pragma unroll
+      for (int u = 0; u < kAlignIds; ++u) {
+        const int f = base0 + 64 * u + lane;  // < hi where eb[u] >= 0
+        if (eb[u] >= 0) scratch[f] += cnt[w][eb[u]];
+      }
+    }
+  }
 }
 
 // Block order for the grouped GEMMs, heaviest first: border[r] = the r-th align block sorted by
@@ -381,7 +416,7 @@ hipError_t launch_align(const int32_t* topk_ids, int T, int top_k, int E, int ha
   int CH = 0;
   const int nchunks = align_chunks(T, top_k, E, has_shared, BM, cap, scratch != nullptr, &CH);
   if (nchunks > 0 && scratch) {
-    hipLaunchKernelGGL(align_chunk_kernel, dim3(nchunks), dim3(64), 0, stream, topk_ids, T,
+    hipLaunchKernelGGL(align_chunk_kernel, dim3(nchunks), dim3(64 * kChunkWaves), 0, stream, topk_ids, T,
                        top_k, E, has_shared, CH, scratch);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -391,7 +426,7 @@ hipError_t launch_align(const int32_t* topk_ids, int T, int top_k, int E, int ha
     return hipGetLastError();
   }
   if (nchunks > 0) {
-    hipLaunchKernelGGL(align_chunk_kernel, dim3(nchunks), dim3(64), 0, stream, topk_ids, T,
+    hipLaunchKernelGGL(align_chunk_kernel, dim3(nchunks), dim3(64 * kChunkWaves), 0, stream, topk_ids, T,
                        top_k, E, has_shared, CH, sorted);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;

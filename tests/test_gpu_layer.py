@@ -395,6 +395,29 @@ def test_fused_prefill_align_layout(shared):
     assert list(got_border) == want
 
 
+@pytest.mark.parametrize("T,k,E", [(300, 8, 256),     # part of the chunk's waves without slots
+                                   (2200, 64, 64)])   # 140 800 slots: more than a wave holds
+def test_prefill_align_chunk_waves(T, k, E):
+    """The chunk ranks of the large-input align at both ends of a wave's share of a chunk."""
+    _say(f"prefill align chunk waves T={T} k={k} E={E}")
+    BM = ops.PREFILL_BLOCK_M
+    layer = to_gpu(synth.make_layer(6, num_experts=E, hidden=512, intermediate=256, zipf=True))
+    x = synth.make_tokens(T, 512, seed=14).cuda()
+    ws = torch.full((ops.workspace_bytes(T, k, layer.experts, False, "prefill"),), 0x5A,
+                    dtype=torch.uint8, device="cuda")
+    _, ids, _ = ops.moe_layer(x, layer.router_w, layer.experts, top_k=k,
+                              logit_bias=layer.logit_bias, path="prefill", workspace=ws,
+                              return_routing=True)
+    torch.cuda.synchronize()
+    cap = ops.capacity_blocks(T, k, E, False, BM)
+    o = _workspace_offsets(T, k, E, False, BM, cap)
+    i32 = ws.view(torch.int32).cpu().numpy()
+    rs, re_, rn = moe_ref.align_block_padded(ids.cpu().numpy(), E, BM, capacity_blocks=cap)
+    assert int(i32[o["ntpp"] // 4]) == rn
+    assert np.array_equal(i32[o["sorted"] // 4: o["sorted"] // 4 + cap * BM], rs)
+    assert np.array_equal(i32[o["eids"] // 4: o["eids"] // 4 + cap], re_)
+
+
 @pytest.mark.parametrize("T", [8, 64])
 def test_config2_zipf_decode_full_shape(T):
     """Config 2 at full shape with the Zipf(1.1) routing skew, decode path, against the oracle
