@@ -3,12 +3,12 @@
 // combination logits = prior + scale * residual (train_hidden_residual_predictor_smoke.py:446)
 // and the top-k experts of every (example, future delta):
 //
-//   z  = bf16(x . W_enc^T + b_enc)                    encoder Linear (canonical fp32 dot)
+//   z  = bf16(x . W_enc^T + b_enc)                    encoder Linear (fp32 sums)
 //   a  = bf16(silu(z))                                SiLU
 //   s  = bf16(LayerNorm(a) * ln_w + ln_b)             LayerNorm over the width (fp32 statistics)
 //   c_d = bf16(bf16(s + E_layer[layer]) + E_delta[d]) context per future delta d
 //   g_d = bf16(silu(c_d))
-//   r_d = g_d . W_cls^T + b_cls                       classifier (canonical fp32 dot), fp32
+//   r_d = g_d . W_cls^T + b_cls                       classifier (fp32 sums), fp32
 //   out_d = prior_d + scale * r_d                     (prior optional), top-k by (value, id)
 //
 // Every Linear input is bf16 (the dtype of a bf16 model's activations), so the products of the
