@@ -163,10 +163,11 @@ enum Routing {
 
 // [align ->] W1 -> W2 -> top-k sum over a workspace. ids [T * top_k] and w [T * top_k (+ T shared
 // gates)] are the routing: the workspace's own, or a caller's arrays (read only: every form but
-// ROUTE_GRID_LOGITS, which publishes its top-k to them).
+// ROUTE_GRID_LOGITS, which publishes its top-k to them). given: the ids are a caller's and may
+// name no expert; the router's own are all in [0, E).
 int run_experts(const uint16_t* x, int T, int top_k, const moe_expert_set_v1* ex,
                 const moe_expert_set_v1* sh, const Workspace& L, void* ws, int32_t* ids, float* w,
-                uint16_t* out, int path, Routing routing, hipStream_t stream) {
+                bool given, uint16_t* out, int path, Routing routing, hipStream_t stream) {
   const int has_shared = sh ? 1 : 0;
   const ExpertsDev ed = make_experts_dev(ex, sh);
   SlotsDev sd{T, top_k, T * top_k + (has_shared ? T : 0)};
@@ -185,6 +186,8 @@ int run_experts(const uint16_t* x, int T, int top_k, const moe_expert_set_v1* ex
   }
   int32_t* border =
       routing == ROUTE_ALIGN && path == MOE_PATH_PREFILL ? at<int32_t>(ws, L.border) : nullptr;
+  // The sum looks at the ids only where a slot can be dropped.
+  const int32_t* drop_ids = given || ex->expert_row ? ids : nullptr;
   const bool grid = routing == ROUTE_GRID_LOGITS || routing == ROUTE_GRID_IDS;
   if (grid) {
     const SlotGrid sg{1, routing == ROUTE_GRID_LOGITS ? at<float>(ws, L.logits) : nullptr, ids, w};
@@ -215,7 +218,7 @@ int run_experts(const uint16_t* x, int T, int top_k, const moe_expert_set_v1* ex
     uint16_t* ys16 = at<uint16_t>(ws, L.ys);
     MOE_CHECK_HIP(launch_w2_prefill_bf16(h, ed, sd, sorted, eids, ntpp, border, L.bm, L.cap, w, ys16,
                                          stream), "w2");
-    MOE_CHECK_HIP(launch_moe_sum_bf16(ys16, T, top_k, ex->hidden, has_shared, ids,
+    MOE_CHECK_HIP(launch_moe_sum_bf16(ys16, T, top_k, ex->hidden, has_shared, drop_ids,
                                       ex->num_experts, ex->expert_row, out, stream),
                   "moe_sum");
     return MOE_OK;
@@ -227,8 +230,8 @@ int run_experts(const uint16_t* x, int T, int top_k, const moe_expert_set_v1* ex
     MOE_CHECK_HIP(dispatch_w2(path, h, ed, sd, sorted, eids, ntpp, nullptr, L.bm, L.cap, w, ys,
                               stream),
                   "w2");
-  MOE_CHECK_HIP(launch_moe_sum(ys, T, top_k, ex->hidden, has_shared, ids, ex->num_experts,
-                               ex->expert_row, out, stream),
+  MOE_CHECK_HIP(launch_moe_sum(ys, T, top_k, ex->hidden, has_shared, drop_ids, ex->num_experts,
+                               ex->expert_row, true, out, stream),
                 "moe_sum");
   return MOE_OK;
 }
@@ -429,7 +432,7 @@ int moe_sum_v1(const float* ys, int32_t T, int32_t top_k, int32_t hidden, int32_
   if (T == 0) return MOE_OK;
   if (!ys || !out || !topk_ids) return fail(MOE_ERR_NULL, "moe_sum: NULL pointer");
   MOE_CHECK_HIP(launch_moe_sum(ys, T, top_k, hidden, has_shared ? 1 : 0, topk_ids, num_experts,
-                               expert_row, out, (hipStream_t)stream),
+                               expert_row, false, out, (hipStream_t)stream),
                 "moe_sum");
   return MOE_OK;
 }
@@ -531,7 +534,8 @@ int layer_impl(const uint16_t* x, int32_t T, const uint16_t* router_w, const flo
                                         shared ? shared_gate_w : nullptr, logit_bias, top_k,
                                         logits, at<float>(workspace, L.norms), ids, w, s),
                   "router (prefill)");
-    rc = run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, out, path, ROUTE_ALIGN, s);
+    rc = run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, false, out, path,
+                     ROUTE_ALIGN, s);
     if (rc) return rc;
     return copy_routing(ids, w, T, top_k, topk_ids_out, topk_weights_out, s);
   }
@@ -565,7 +569,8 @@ int layer_impl(const uint16_t* x, int32_t T, const uint16_t* router_w, const flo
     MOE_CHECK_HIP(launch_router_topk(logits, T, E, top_k, shared ? 1 : 0, ids, w, s),
                   "router topk");
   }
-  rc = run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, out, path, routing, s);
+  rc = run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, false, out, path, routing,
+                   s);
   if (rc) return rc;
   return copy_routing(ids, w, T, top_k, topk_ids_out, topk_weights_out, s);
 }
@@ -672,7 +677,8 @@ int moe_fused_experts_v1(const uint16_t* x, int32_t T, const int32_t* topk_ids,
   const Routing routing = (path == MOE_PATH_DECODE && slot_grid_fits(T, top_k, shared ? 1 : 0))
                               ? ROUTE_GRID_IDS
                               : ROUTE_ALIGN;
-  return run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, out, path, routing, s);
+  return run_experts(x, T, top_k, experts, shared, L, workspace, ids, w, true, out, path, routing,
+                     s);
 }
 
 }  // extern "C"
@@ -772,7 +778,8 @@ int moe_offload_layer_v1(uint64_t cache, int32_t layer, const uint16_t* x, int32
   if (rc) return rc;
   const Routing routing =
       (path == MOE_PATH_DECODE && slot_grid_fits(T, top_k, 0)) ? ROUTE_GRID_IDS : ROUTE_ALIGN;
-  rc = run_experts(x, T, top_k, experts, nullptr, L, workspace, ids, w, out, path, routing, s);
+  rc = run_experts(x, T, top_k, experts, nullptr, L, workspace, ids, w, false, out, path, routing,
+                   s);
   if (rc) return rc;
   // The wait for the ids drained the compute stream, and the demand's slots (the only ones the
   // kernels just enqueued read) stay pinned until layer_done: the prefetch needs no ordering

@@ -118,9 +118,11 @@ hipError_t launch_w2_decode_slotgrid(const uint16_t* h, const ExpertsDev& ed, co
                                      const SlotGrid& sg, float* ys, hipStream_t stream);
 
 // ids == nullptr: every slot is summed; otherwise routed slots with a dropped expert are skipped.
+// own_rows: ys holds a row for every slot that may be read (its values do not count where the
+// slot is dropped); without it a dropped slot's row is never read.
 hipError_t launch_moe_sum(const float* ys, int T, int top_k, int H, int has_shared,
                           const int32_t* ids, int num_experts, const int32_t* expert_row,
-                          uint16_t* out, hipStream_t stream);
+                          bool own_rows, uint16_t* out, hipStream_t stream);
 // moe_sum over bf16 slot rows (summed in fp32 in slot order).
 hipError_t launch_moe_sum_bf16(const uint16_t* ys, int T, int top_k, int H, int has_shared,
                                const int32_t* ids, int num_experts, const int32_t* expert_row,

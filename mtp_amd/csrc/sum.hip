@@ -10,13 +10,13 @@ namespace {
 // fp32 (YT = float) or bf16 (YT = uint16_t). With `ids`, routed slots whose expert is dropped
 // (routed_ok false: their ys rows were never written) are skipped.
 // Each thread sums 16 bytes of columns (4 fp32 or 8 bf16). Slots are taken TK at a time: all
-// loads of a chunk are issued together (a slot past top_k reads zeros without a memory access),
-// the ids and the expert rows beside them and not before them, so a decode batch, which latency
-// bounds, waits for one memory latency instead of three (eight layers of 48 tokens, hidden 1024:
-// 163 -> 160 us); a dropped slot's row is masked to +0 after the load, which leaves the running
-// sum unchanged. With UNIFORM (a token's columns cover whole waves) the token
-// index is wave-uniform and its ids and expert rows are scalar loads, leaving the vector memory
-// pipeline to the slot rows.
+// loads of a chunk are issued together (a slot past top_k or a dropped one reads zeros without a
+// memory access, and +0 leaves the running sum unchanged), so a chunk waits for the memory latencies
+// of its ids, its expert rows and its slot rows instead of one per slot. With BESIDE the slot rows
+// are loaded ahead of the wait for the ids, also those of dropped slots, which are masked to +0
+// afterwards: one latency instead of three. With UNIFORM (a token's columns cover whole waves)
+// the token index is wave-uniform and its ids and expert rows are scalar loads, leaving the vector
+// memory pipeline to the slot rows.
 template <typename YT>
 struct SumVec {
   static constexpr int N = 16 / sizeof(YT);  // columns per thread
@@ -40,7 +40,7 @@ MOE_DEV SumVec<YT> ys_vec(u32x4 d, bool ok) {
   return o;
 }
 
-template <int TK, typename YT, bool UNIFORM>
+template <int TK, typename YT, bool UNIFORM, bool BESIDE>
 __global__ __launch_bounds__(256) void moe_sum_kernel(const YT* __restrict__ ys, int T, int top_k,
                                                       int H, int has_shared,
                                                       const int32_t* __restrict__ ids,
@@ -73,9 +73,9 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const YT* __restrict__ ys,
 #pragma unroll
     for (int i = 0; i < TK; ++i) {
       ok[i] = i0 + i < top_k;
-      d[i] = load_row(t * top_k + i0 + i, ok[i]);
+      if constexpr (BESIDE) d[i] = load_row(t * top_k + i0 + i, ok[i]);
     }
-    __builtin_amdgcn_sched_barrier(0);  // the rows' loads ahead of the wait for the ids
+    if constexpr (BESIDE) __builtin_amdgcn_sched_barrier(0);  // rows ahead of the wait for the ids
     if (ids) {
       int e[TK];
       if constexpr (UNIFORM) {  // wave-uniform: scalar loads
@@ -102,9 +102,13 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const YT* __restrict__ ys,
         for (int i = 0; i < TK; ++i) ok[i] = ok[i] && r[i] >= 0;
       }
     }
+    if constexpr (!BESIDE) {
+#pragma unroll
+      for (int i = 0; i < TK; ++i) d[i] = load_row(t * top_k + i0 + i, ok[i]);
+    }
 #pragma unroll
     for (int i = 0; i < TK; ++i) {
-      const SumVec<YT> v = ys_vec<YT>(d[i], ok[i]);
+      const SumVec<YT> v = ys_vec<YT>(d[i], !BESIDE || ok[i]);
 #pragma unroll
       for (int j = 0; j < N; ++j) s[j] += v.v[j];
     }
@@ -127,37 +131,49 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const YT* __restrict__ ys,
 template <typename YT, bool UNIFORM>
 hipError_t launch_moe_sum_u(const YT* ys, int T, int top_k, int H, int has_shared,
                             const int32_t* ids, int num_experts, const int32_t* expert_row,
-                            uint16_t* out, hipStream_t stream) {
+                            bool own_rows, uint16_t* out, hipStream_t stream) {
   const int64_t n = (int64_t)T * (H / SumVec<YT>::N);
   // Few threads: one wave per workgroup, so that they spread over all 256 CUs.
   const int block = n <= 256 * 256 ? 64 : 256;
   const dim3 grid((unsigned)((n + block - 1) / block));
-#define MOE_SUM_CASE(TKV)                                                                      \
-  if (top_k <= TKV) {                                                                          \
-    hipLaunchKernelGGL((moe_sum_kernel<TKV, YT, UNIFORM>), grid, dim3(block), 0, stream, ys, T, \
-                       top_k, H, has_shared, ids, num_experts, expert_row, out);               \
-    return hipGetLastError();                                                                  \
+  // BESIDE where latency bounds the sum and the caller has a row for every slot, dropped or not:
+  // up to 128 workgroups of rows it costs nothing even if every slot is dropped (eight routed
+  // layers of 48 tokens, hidden 1024: 163 -> 160 us); beyond, a dropped slot's row is
+  // traffic that the ids save (1024 tokens, top-8, hidden 2048, half of the slots dropped: 8.1
+  // against 12.1 us; 8192 tokens 44 against 103).
+  [[maybe_unused]] const bool beside = own_rows && ids && n <= 128 * 256;
+#define MOE_SUM_GO(TKV, B)                                                                      \
+  {                                                                                             \
+    hipLaunchKernelGGL((moe_sum_kernel<TKV, YT, UNIFORM, B>), grid, dim3(block), 0, stream, ys, \
+                       T, top_k, H, has_shared, ids, num_experts, expert_row, out);             \
+    return hipGetLastError();                                                                   \
+  }
+#define MOE_SUM_CASE(TKV)                                   \
+  if (top_k <= TKV) {                                       \
+    if constexpr (sizeof(YT) == 4) {                        \
+      if (beside) MOE_SUM_GO(TKV, true)                     \
+    }                                                       \
+    MOE_SUM_GO(TKV, false)                                  \
   }
   MOE_SUM_CASE(1) MOE_SUM_CASE(2) MOE_SUM_CASE(4) MOE_SUM_CASE(8)
+  MOE_SUM_GO(16, false)
 #undef MOE_SUM_CASE
-  hipLaunchKernelGGL((moe_sum_kernel<16, YT, UNIFORM>), grid, dim3(block), 0, stream, ys, T, top_k,
-                     H, has_shared, ids, num_experts, expert_row, out);
-  return hipGetLastError();
+#undef MOE_SUM_GO
 }
 
 template <typename YT>
 hipError_t launch_moe_sum_t(const YT* ys, int T, int top_k, int H, int has_shared,
                             const int32_t* ids, int num_experts, const int32_t* expert_row,
-                            uint16_t* out, hipStream_t stream) {
+                            bool own_rows, uint16_t* out, hipStream_t stream) {
   constexpr int N = SumVec<YT>::N;
   if ((int64_t)T * H == 0) return hipSuccess;
   if (H % N != 0) return hipErrorInvalidValue;
   if ((int64_t)(T * top_k + T) * H * (int64_t)sizeof(YT) >= kOutOfRange) return hipErrorInvalidValue;
   if ((H / N) % 64 == 0)  // a token's columns cover whole waves
     return launch_moe_sum_u<YT, true>(ys, T, top_k, H, has_shared, ids, num_experts, expert_row,
-                                      out, stream);
+                                      own_rows, out, stream);
   return launch_moe_sum_u<YT, false>(ys, T, top_k, H, has_shared, ids, num_experts, expert_row,
-                                     out, stream);
+                                     own_rows, out, stream);
 }
 
 // Sum of the fused W1+W2 partial rows (gemm_decode_kernel FW2): out[t][n] = bf16 of the fp32
@@ -231,14 +247,14 @@ hipError_t launch_partial_sum(const float* part, int T, int top_k, int H, int nc
 
 hipError_t launch_moe_sum(const float* ys, int T, int top_k, int H, int has_shared,
                           const int32_t* ids, int num_experts, const int32_t* expert_row,
-                          uint16_t* out, hipStream_t stream) {
-  return launch_moe_sum_t<float>(ys, T, top_k, H, has_shared, ids, num_experts, expert_row, out,
-                                 stream);
+                          bool own_rows, uint16_t* out, hipStream_t stream) {
+  return launch_moe_sum_t<float>(ys, T, top_k, H, has_shared, ids, num_experts, expert_row,
+                                 own_rows, out, stream);
 }
 
 hipError_t launch_moe_sum_bf16(const uint16_t* ys, int T, int top_k, int H, int has_shared,
                                const int32_t* ids, int num_experts, const int32_t* expert_row,
                                uint16_t* out, hipStream_t stream) {
   return launch_moe_sum_t<uint16_t>(ys, T, top_k, H, has_shared, ids, num_experts, expert_row,
-                                    out, stream);
+                                    false, out, stream);
 }

@@ -194,6 +194,35 @@ def test_align_known_answer():
     assert s.cpu().tolist()[:12] == [0, 3, 3, 3, 1, 3, 3, 3, 2, 3, 3, 3]
 
 
+def test_dropped_rows_are_not_read_by_the_sum():
+    """A dropped slot's ys row is never read: the sum of a batch whose slots are all dropped leaves
+    the 0.5 GB of rows alone. With every row read it takes as long as a batch without drops; the
+    ids and the output are a tenth of that traffic."""
+    _say("moe_sum traffic of dropped slots")
+    T, k, H = 8192, 8, 2048
+    experts = synth.make_layer(1, num_experts=16, hidden=512, intermediate=256, device="cuda").experts
+    ys = torch.randn(T * k, H, device="cuda")
+    kept = torch.arange(T * k, device="cuda", dtype=torch.int32).view(T, k) % 16
+
+    def ms(ids):
+        best = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                out = ops.moe_sum(ys, ids, experts)
+            b.record()
+            torch.cuda.synchronize()
+            best.append(a.elapsed_time(b))
+        return min(best), out
+
+    full, _ = ms(kept)
+    none, out = ms(torch.full_like(kept, -1))
+    print(f"  kept {full / 20 * 1e3:.1f} us, dropped {none / 20 * 1e3:.1f} us", flush=True)
+    assert not out.any()
+    assert none < 0.7 * full
+
+
 @pytest.mark.parametrize("path", ["decode", "prefill"])
 def test_stepwise_entry_points_with_dropped_ids_and_poisoned_ys(path):
     """align -> W1 -> W2 -> moe_sum as separate entry points, with ids outside [0, E) and a ys
