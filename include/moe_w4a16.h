@@ -227,7 +227,9 @@ int moe_layer_noalloc_v1(const uint16_t* x, int32_t T, const uint16_t* router_w,
  * and moe_tokens with given ids (src/mtp_expert_prefetch/mtp/extra_tensors.py:544-598).
  * A slot is dropped (contributes zero) when its id is outside [0, num_experts) or, with an
  * expert_row map, names an expert whose row is negative (not resident), as the reference drops
- * ids outside [0, E) and unmapped experts (vllm_router_trace.py:14138-14153). */
+ * ids outside [0, E) and unmapped experts (vllm_router_trace.py:14138-14153).
+ * topk_ids and topk_weights are read until the call's last kernel and are not written; they may
+ * lie inside out or inside the workspace (the call then copies them first). */
 int moe_fused_experts_v1(const uint16_t* x, int32_t T, const int32_t* topk_ids,
                          const float* topk_weights, int32_t top_k,
                          const moe_expert_set_v1* experts, const moe_expert_set_v1* shared,

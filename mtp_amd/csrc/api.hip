@@ -649,14 +649,18 @@ int moe_fused_experts_v1(const uint16_t* x, int32_t T, const int32_t* topk_ids,
   // The kernels read the caller's routing in place (copied to the workspace first it cost two
   // launches: eight routed layers of 48 tokens, hidden 1024, 197 -> 169 us). With a shared
   // expert its gate kernel writes the gates behind the routed weights, so those move to the
-  // workspace in that launch. A routing that shares bytes with the output, which the last kernels
-  // write while others still read the routing, is copied as a whole.
+  // workspace in that launch. A routing that shares bytes with the output or with the workspace,
+  // which kernels of the call write while later ones still read the routing, is copied as a whole.
   const size_t n = (size_t)T * top_k;
-  auto in_out = [&](const void* p, size_t bytes) {
-    const uintptr_t a = (uintptr_t)p, o = (uintptr_t)out;
-    return a < o + (size_t)T * experts->hidden * 2 && o < a + bytes;
+  auto overlaps = [](const void* p, size_t bytes, const void* q, size_t q_bytes) {
+    const uintptr_t a = (uintptr_t)p, b = (uintptr_t)q;
+    return a < b + q_bytes && b < a + bytes;
   };
-  const bool copy = in_out(topk_ids, n * 4) || in_out(topk_weights, n * 4);
+  auto written = [&](const void* p) {
+    return overlaps(p, n * 4, out, (size_t)T * experts->hidden * 2) ||
+           overlaps(p, n * 4, workspace, L.total);
+  };
+  const bool copy = written(topk_ids) || written(topk_weights);
   int32_t* ids = const_cast<int32_t*>(topk_ids);
   float* w = const_cast<float*>(topk_weights);
   if (copy) {

@@ -205,6 +205,37 @@ def test_given_routing_is_read_in_place(T, path, with_shared, aliased):
     assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("section", ["h", "ys"])  # written by W1 and by W2
+@pytest.mark.parametrize("T,path", [(2, "decode"), (40, "decode"), (40, "prefill")])
+def test_given_routing_inside_the_workspace(T, path, section):
+    """Routing that lies in a section of the workspace that W1 or W2 writes is copied before them:
+    the output is that of the same routing in arrays of its own."""
+    import ctypes
+
+    from mtp_amd import _lib
+    _say(f"given routing in the workspace T={T} {path} {section}")
+    g = to_gpu(small_layer(3))
+    x, k, E = synth.make_tokens(T, 512, seed=T).cuda(), 4, 16
+    want, ids, w = ops.moe_layer(x, g.router_w, g.experts, top_k=k, path=path, return_routing=True)
+    assert torch.equal(ops.fused_experts(x, ids, w, g.experts, path=path), want)
+    bm = ops.PREFILL_BLOCK_M if path == "prefill" else ops.DECODE_BLOCK_M
+    cap = ops.capacity_blocks(T, k, E, False, bm)
+    border = _workspace_offsets(T, k, E, False, bm, cap)["border"] // 4  # h follows it
+    ws = torch.empty(ops.workspace_bytes(T, k, g.experts, False, path), dtype=torch.uint8,
+                     device="cuda")
+    flat, n = ws.view(torch.int32), T * k
+    first = border + -(-cap // 64) * 64 if section == "h" else flat.numel() - 2 * n
+    flat[first:first + n] = ids.view(-1)
+    flat[first + n:first + 2 * n] = w.view(-1).view(torch.int32)
+    out, p = torch.empty_like(x), {"decode": 1, "prefill": 2}[path]
+    ex = g.experts.struct()
+    _lib.check(_lib.load().moe_fused_experts_v1(
+        x.data_ptr(), T, flat[first:].data_ptr(), flat[first + n:].data_ptr(), k, ctypes.byref(ex),
+        None, None, ws.data_ptr(), ws.numel(), out.data_ptr(), p,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert torch.equal(out, want)
+
+
 def test_empty_batch_gives_empty_outputs():
     """A batch of no tokens is a no-op of every layer entry point (T = 0 returns at once; align
     writes only ntpp = 0 and takes NULL tables); the shapes come back empty."""
