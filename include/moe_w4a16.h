@@ -282,8 +282,8 @@ int64_t moe_hr_predictor_workspace_bytes_v1(int32_t N, const moe_hr_predictor_pa
  * (train_hidden_residual_predictor_smoke.py:446; prior NULL = 0; scale = scale_per_example[n]
  * when given, else residual_scale, as apply_residual_scale :108-121 with a fixed or learnt
  * gamma), and the top_k experts of every (example, delta) row by (value, lower id).
- * Activations between the Linear layers are bf16; the dot products use the router's canonical
- * fp32 order. A layer id outside [0, num_layers) reads a zero embedding. logits_out: NULL or
+ * Activations between the Linear layers are bf16; the dot products are fp32 sums of exact
+ * products, in an order that depends on N, future_window, width and num_experts. A layer id outside [0, num_layers) reads a zero embedding. logits_out: NULL or
  * fp32 [N, future_window, num_experts]; topk_ids int32 [N, future_window, top_k]. */
 int moe_hr_predictor_v1(const uint16_t* hidden, int32_t N, const int32_t* layer_ids,
                         const moe_hr_predictor_params_v1* params, const float* prior,

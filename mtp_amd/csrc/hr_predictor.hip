@@ -11,14 +11,19 @@
 //   r_d = g_d . W_cls^T + b_cls                       classifier (fp32 sums), fp32
 //   out_d = prior_d + scale * r_d                     (prior optional), top-k by (value, id)
 //
-// Every Linear input is bf16 (the dtype of a bf16 model's activations), so the products of the
-// two Linear layers run on v_mfma_f32_16x16x32_bf16 with fp32 sums. Two launches: the encoder
-// (hr_encoder_kernel), then everything per 16 context rows (hr_rows_kernel). At these sizes a call
-// is bound by launches and by each kernel's chain of loads, not by bytes or arithmetic: 160
-// examples of the default shape (hidden 2048, width 256, 4 deltas, 256 experts, top-16) took 53.5 us
-// in four launches with both products on the VALU (the classifier alone 36 us), and take 21.4 us now;
-// the error against 64 bits is the same (3.7e-3 to 4.2e-3 of the residual over 3 to 640 examples and
-// widths 128 to 512: the bf16 activations).
+// Every Linear input is bf16 (the dtype of a bf16 model's activations), and both Linear layers sum
+// exact products in fp32, on v_mfma_f32_16x16x32_bf16 or in the router's canonical order
+// (routing.h:logits_tile). At these sizes a call is bound by launches and by each kernel's chain
+// of loads, not by bytes or arithmetic. Two forms (hr_split chooses):
+//  - two launches: the encoder, then everything per 16 context rows (hr_rows_kernel). Each of its
+//    workgroups reads the whole classifier, so it is the form for many rows or a small classifier:
+//    160 examples of the default shape (hidden 2048, width 256, 4 deltas, 256 experts, top-16)
+//    21.4 us, in the other form with the canonical encoder 53.5;
+//  - four launches for few rows of a large classifier: the encoder, the context rows, the
+//    classifier over many workgroups, the selection: one example and delta of width 256 13.6 us
+//    (17.2 in the other form), of width 512 14.4 (25.8), of width 1024 and 512 experts 20 (55).
+// The error against 64 bits is the same (3.7e-3 to 4.2e-3 of the residual over 3 to 640 examples
+// and widths 128 to 512: the bf16 activations).
 #include <math.h>
 #include <stdio.h>
 
@@ -36,6 +41,9 @@ MOE_DEV f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
 MOE_DEV float bf16_round(float v) { return bf16_to_f32(f32_to_bf16_rne(v)); }
 
 constexpr int kMaxWidth = 1024;
+// Up to this many examples the encoder runs as the router's GEMV: a 16-row MFMA tile would be
+// partly padding (width 256: 1 example 3.3 against 4.9 us, 16 examples 4.9 against 6.0, 40 the same).
+constexpr int kEncFew = 16;
 
 // z[n][j] = x_n . W_enc[j] (fp32): a 16 x 16 (example x output) tile per workgroup, its four waves a
 // quarter of K each (added in wave order). A wave has 16 k-steps of both operands in flight at
@@ -79,7 +87,7 @@ __global__ __launch_bounds__(64 * kEncWaves) void hr_encoder_kernel(
 #pragma unroll
   for (int i = 0; i < 4; ++i) {  // D[4 kq + i][r]
     const int n = n0 + 4 * kq + i, j = j0 + r;
-    if (n < N && j < W) z[(int64_t)n * W + j] = acc[i];
+    if (n < N && j < W) z[(int64_t)n * (W + 1) + j] = acc[i];
   }
 }
 
@@ -134,7 +142,7 @@ __global__ __launch_bounds__(64 * kRows) void hr_rows_kernel(
 
   // context row (lane: columns lane + 64 i); columns past the width hold zeros
   float a[NC], sum = 0.0f;
-  const __amdgpu_buffer_rsrc_t zr = buf_rsrc(z + (int64_t)n * W, (uint32_t)W * 4u);
+  const __amdgpu_buffer_rsrc_t zr = buf_rsrc(z + (int64_t)n * (W + 1), (uint32_t)W * 4u);
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const int j = lane + 64 * i;
@@ -210,25 +218,159 @@ __global__ __launch_bounds__(64 * kRows) void hr_rows_kernel(
   if (lane < top_k) ids[(int64_t)row * top_k + lane] = my_i;
 }
 
+constexpr int kCtxThreads = 256;
+constexpr int kCtxMaxPerThread = kMaxWidth / kCtxThreads;
+
+// Fixed-order sum over the workgroup: per-thread value -> wave butterfly -> waves in order.
+MOE_DEV float block_sum(float v, float* red) {
+  v = bfly_sum(v);
+  const int wv = threadIdx.x >> 6;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[wv] = v;
+  __syncthreads();
+  float s = 0.0f;
+  for (int w = 0; w < kCtxThreads / 64; ++w) s += red[w];
+  return s;
+}
+
+// One workgroup per example n: the encoder output row z[n] (fp32 dot, stride W + 1) -> the
+// future_window context rows g[n * F + d] (bf16).
+__global__ __launch_bounds__(kCtxThreads) void hr_context_kernel(
+    const float* __restrict__ z, int N, int W, const float* __restrict__ enc_b,
+    const uint16_t* __restrict__ ln_w, const uint16_t* __restrict__ ln_b, float ln_eps,
+    const int32_t* __restrict__ layer_ids, int num_layers, const uint16_t* __restrict__ layer_emb,
+    const uint16_t* __restrict__ delta_emb, int F, uint16_t* __restrict__ g) {
+  __shared__ float red[kCtxThreads / 64];
+  const int n = blockIdx.x;
+  const int tid = threadIdx.x;
+  float a[kCtxMaxPerThread];
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kCtxMaxPerThread; ++i) {
+    const int j = tid + kCtxThreads * i;
+    a[i] = 0.0f;
+    if (j < W) {
+      const float zb = bf16_round(z[(int64_t)n * (W + 1) + j] + enc_b[j]);
+      a[i] = bf16_round(zb / (1.0f + expf(-zb)));
+      sum += a[i];
+    }
+  }
+  const float mean = block_sum(sum, red) / (float)W;
+  float sq = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kCtxMaxPerThread; ++i) {
+    const int j = tid + kCtxThreads * i;
+    if (j < W) {
+      const float d = a[i] - mean;
+      sq = __builtin_fmaf(d, d, sq);
+    }
+  }
+  const float var = block_sum(sq, red) / (float)W;
+  const float rstd = 1.0f / sqrtf(var + ln_eps);
+  const int layer = layer_ids[n];
+  const bool layer_ok = layer >= 0 && layer < num_layers;  // else the embedding reads zeros
+#pragma unroll
+  for (int i = 0; i < kCtxMaxPerThread; ++i) {
+    const int j = tid + kCtxThreads * i;
+    if (j >= W) continue;
+    const float s = bf16_round((a[i] - mean) * rstd * bf16_to_f32(ln_w[j]) + bf16_to_f32(ln_b[j]));
+    const float le = layer_ok ? bf16_to_f32(layer_emb[(int64_t)layer * W + j]) : 0.0f;
+    const float sl = bf16_round(s + le);
+    for (int d = 0; d < F; ++d) {
+      const float c = bf16_round(sl + bf16_to_f32(delta_emb[(int64_t)d * W + j]));
+      g[((int64_t)n * F + d) * W + j] = (uint16_t)f32_to_bf16_rne(c / (1.0f + expf(-c)));
+    }
+  }
+}
+
+// One wave per row r = n * F + d: v = (prior ? prior[r] : 0) + scale_n * logits[r], optionally
+// written to out, and the top-k of v by (value, lower id).
+template <int MAXC>
+__global__ __launch_bounds__(256) void hr_select_kernel(
+    const float* __restrict__ logits, int rows, int F, int E, const float* __restrict__ prior,
+    float scale, const float* __restrict__ scale_per_example, int top_k,
+    float* __restrict__ out, int32_t* __restrict__ ids) {
+  const int lane = threadIdx.x & 63;
+  const int r = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (r >= rows) return;
+  const float sc = scale_per_example ? scale_per_example[r / F] : scale;
+  const __amdgpu_buffer_rsrc_t lr = buf_rsrc(logits + (int64_t)r * (E + 1), (uint32_t)E * 4u);
+  const __amdgpu_buffer_rsrc_t pr = buf_rsrc(prior ? prior + (int64_t)r * E : nullptr,
+                                             prior ? (uint32_t)E * 4u : 0u);
+  uint32_t key[MAXC];
+#pragma unroll
+  for (int c = 0; c < MAXC; ++c) {
+    const int e = lane + 64 * c;
+    const float l = __uint_as_float(buf_ld32(lr, (uint32_t)e * 4u));
+    const float p = __uint_as_float(buf_ld32(pr, (uint32_t)e * 4u));
+    const float v = p + sc * l;
+    if (out && e < E) out[(int64_t)r * E + e] = v;
+    key[c] = topk_ord(v) & (0u - (uint32_t)(e < E));
+  }
+  int my_i;
+  uint32_t my_key;
+  topk_select_keys<MAXC>(key, top_k, lane, my_i, my_key);
+  if (lane < top_k) ids[(int64_t)r * top_k + lane] = my_i;
+}
+
 }  // namespace
 
-// Workspace: z [N][W] fp32.
+namespace {
+int64_t a256(int64_t v) { return (v + 255) & ~int64_t(255); }
+
+// Whether the context rows, the classifier and the selection are launches of their own. Measured
+// over widths 64 to 1024, 64 to 512 experts and 1 to 2048 rows, both forms:
+//  - up to 64 rows (the small tiles of launch_router_logits) beyond width 128 or 256 experts:
+//    4 rows of width 256 15.6 against 18.2 us, 64 rows 19.9 against 22.0; at width 128 and 256
+//    experts they are equal, and the two launches win below;
+//  - up to 1024 rows where the width is a multiple of 512, which the classifier's 8 x 8 tiles
+//    need (width 512: 512 rows 27.4 against 30.8 us; width 384: 46.4 against 27.9).
+bool hr_split(int W, int E, int64_t rows) {
+  return (rows <= 64 && (W > 128 || E > 256)) || (rows <= 1024 && W % 512 == 0);
+}
+}  // namespace
+
+// Workspace sections: z [N][W + 1] fp32; in the split form also g [N * F][W] bf16 and logits
+// [N * F][E + 1] fp32.
 int64_t hr_predictor_workspace(int N, int W, int F, int E) {
-  (void)F;
-  (void)E;
-  return ((int64_t)N * W * 4 + 255) & ~int64_t(255);
+  const int64_t rows = (int64_t)N * F, z = a256((int64_t)N * (W + 1) * 4);
+  return hr_split(W, E, rows) ? z + a256(rows * W * 2) + a256(rows * (E + 1) * 4) : z;
 }
 
 hipError_t launch_hr_predictor(const uint16_t* x, int N, int H, const int32_t* layer_ids,
                                const moe_hr_predictor_params_v1& p, const float* prior, float scale,
                                const float* scale_per_example, int top_k, void* workspace,
                                float* out, int32_t* ids, hipStream_t stream) {
-  const int W = p.width, F = p.future_window, rows = N * F;
-  float* z = static_cast<float*>(workspace);
-  hipLaunchKernelGGL(hr_encoder_kernel, dim3(((N + 15) / 16) * ((W + 15) / 16)),
-                     dim3(64 * kEncWaves), 0, stream, x, N, H, p.enc_w, W, z);
-  const hipError_t err = hipGetLastError();
+  const int W = p.width, F = p.future_window, E = p.num_experts, rows = N * F;
+  char* ws = static_cast<char*>(workspace);
+  float* z = reinterpret_cast<float*>(ws);
+  hipError_t err;
+  if (N <= kEncFew) {
+    err = launch_router_logits(x, N, H, p.enc_w, W, nullptr, nullptr, z, stream);
+  } else {
+    hipLaunchKernelGGL(hr_encoder_kernel, dim3(((N + 15) / 16) * ((W + 15) / 16)),
+                       dim3(64 * kEncWaves), 0, stream, x, N, H, p.enc_w, W, z);
+    err = hipGetLastError();
+  }
   if (err != hipSuccess) return err;
+  if (hr_split(W, E, rows)) {
+    uint16_t* g = reinterpret_cast<uint16_t*>(ws + a256((int64_t)N * (W + 1) * 4));
+    float* lg = reinterpret_cast<float*>(ws + a256((int64_t)N * (W + 1) * 4) +
+                                         a256((int64_t)rows * W * 2));
+    hipLaunchKernelGGL(hr_context_kernel, dim3(N), dim3(kCtxThreads), 0, stream, z, N, W, p.enc_b,
+                       p.ln_w, p.ln_b, p.ln_eps, layer_ids, p.num_layers, p.layer_emb, p.delta_emb,
+                       F, g);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+    // classifier over the context rows, bias added, row stride E + 1
+    err = launch_router_logits(g, rows, W, p.cls_w, E, nullptr, p.cls_b, lg, stream);
+    if (err != hipSuccess) return err;
+    auto select = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((rows + 3) / 4), dim3(256), 0, stream, lg, rows, F, E, prior,
+                         scale, scale_per_example, top_k, out, ids);
+      return hipGetLastError();
+    };
+    return E <= 256 ? select(hr_select_kernel<4>) : select(hr_select_kernel<8>);
+  }
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((rows + kRows - 1) / kRows), dim3(64 * kRows), 0, stream, z,
                        rows, F, layer_ids, p, prior, scale, scale_per_example, top_k, out, ids);
@@ -260,7 +402,7 @@ int hr_check(int32_t N, const moe_hr_predictor_params_v1* p, int32_t top_k) {
       top_k > 64)
     return hr_fail(MOE_ERR_SHAPE, "num_experts in [1, 512] and top_k in [1, min(E, 64)]");
   if (!(p->ln_eps >= 0.0f)) return hr_fail(MOE_ERR_SHAPE, "ln_eps must be >= 0");
-  // 32-bit buffer offsets of the GEMVs
+  // 32-bit offsets of the buffers and of the workspace's sections
   const int64_t lim = int64_t(1) << 31;
   if ((int64_t)N * p->hidden * 2 >= lim || (int64_t)p->width * p->hidden * 2 >= lim ||
       (int64_t)N * p->future_window * p->width * 2 >= lim ||

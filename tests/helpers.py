@@ -38,3 +38,24 @@ def small_layer(layer: int = 0, *, E: int = 16, H: int = 512, I: int = 256, zipf
 
 def to_gpu(layer: synth.SyntheticLayer) -> synth.SyntheticLayer:
     return synth.layer_to(layer, "cuda")
+
+
+def graph_us(fn, calls: int = 10, blocks: int = 9) -> float:
+    """Microseconds of one call of ``fn`` on the GPU alone: the least of several blocks of replays
+    of a graph that holds ``calls`` calls."""
+    fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(calls):
+            fn()
+    best = float("inf")
+    for _ in range(blocks):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            graph.replay()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / (5 * calls))
+    return best

@@ -418,7 +418,9 @@ def test_hidden_residual_predictor_matches_oracle(scope):
 # inside a 32-k step, a 64-lane column and a 16-expert tile; the widest context, 512 experts
 @pytest.mark.parametrize("N,H,W,F,E,k", [(1, 64, 64, 1, 4, 2), (17, 520, 264, 3, 260, 16),
                                          (11, 2048, 72, 3, 40, 8), (6, 1024, 1024, 7, 512, 64),
-                                         (40, 2056, 256, 1, 100, 1)])
+                                         (40, 2056, 256, 1, 100, 1),
+                                         # the same in rows of the two-launch form
+                                         (31, 520, 264, 3, 260, 16), (150, 1024, 1024, 7, 512, 64)])
 def test_hidden_residual_predictor_tile_edges(N, H, W, F, E, k):
     from mtp_amd.predictor import HiddenResidualExpertPredictor
     _say(f"hidden-residual predictor N={N} H={H} W={W} F={F} E={E} k={k}")
@@ -435,6 +437,45 @@ def test_hidden_residual_predictor_tile_edges(N, H, W, F, E, k):
     # classifier's scale) moves a logit; the default shape's tolerance
     assert np.max(np.abs(out.cpu().numpy() - r_out)) <= 1e-2
     _ids_match_up_to_near_ties(ids.cpu().numpy(), r_ids, r_out, 2e-2)
+
+
+# (N, W, F, E): the last row count of the four-launch form, by width and by experts; the last of
+# the widths whose classifier takes 8 x 8 tiles; the last example of the GEMV encoder
+@pytest.mark.parametrize("N,W,F,E", [(64, 256, 1, 256), (32, 128, 2, 300), (256, 512, 4, 64),
+                                     (16, 64, 1, 64)])
+def test_hidden_residual_predictor_forms_agree(N, W, F, E):
+    """An example's logits and experts are the same, up to the order of the fp32 sums, on both
+    sides of a size at which the call takes other kernels."""
+    from mtp_amd.predictor import HiddenResidualExpertPredictor
+    _say(f"hidden-residual predictor forms N={N} W={W} F={F} E={E}")
+    m = HiddenResidualExpertPredictor(hidden_size=1024, num_experts=E, num_layers=5,
+                                      future_window=F, width=W, seed=2, device="cuda")
+    g = torch.Generator().manual_seed(W)
+    h = torch.randn(N + 1, 1024, generator=g).to(torch.bfloat16).cuda()
+    lid = (torch.arange(N + 1) % 5).to(torch.int32)
+    ids0, out0 = m.predict_topk(h[:N], layer_ids=lid[:N], k=8, return_logits=True)
+    ids1, out1 = m.predict_topk(h, layer_ids=lid, k=8, return_logits=True)
+    # the tolerance of the edges' test: an activation may round the other way
+    assert (out1[:N] - out0).abs().max() <= 1e-2
+    _ids_match_up_to_near_ties(ids1[:N].cpu().numpy(), ids0.cpu().numpy(), out0.cpu().numpy(), 2e-2)
+
+
+@pytest.mark.parametrize("W,E", [(512, 256), (1024, 512)])
+def test_one_example_is_not_priced_as_many(W, E):
+    """One row of a wide classifier is spread over the chip: a call costs under half of 512 examples
+    (2048 rows), which read the same weights (measured 0.40 and 0.25 of them; 0.63 and 0.60 where
+    one workgroup reads the whole classifier)."""
+    from mtp_amd.predictor import HiddenResidualExpertPredictor
+    from tests.helpers import graph_us
+    m = HiddenResidualExpertPredictor(hidden_size=2048, num_experts=E, num_layers=40,
+                                      future_window=4, width=W, seed=1, device="cuda")
+    us = {}
+    for N in (1, 512):
+        h = torch.randn(N, 2048, device="cuda").to(torch.bfloat16)
+        lid = torch.arange(N, device="cuda", dtype=torch.int32) % 40
+        us[N] = graph_us(lambda: m.predict_topk(h, layer_ids=lid, k=16))
+    _say(f"hidden-residual predictor W={W} E={E}: {us}")
+    assert us[1] < 0.5 * us[512]
 
 
 def test_hidden_residual_predictor_loads_a_reference_state_dict():
