@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void dequant_tile_kernel(ProjDev p,
   }
 }
 
-// Any group size, group count and base alignment: one thread per packed word.
+// Any group size, group count and base alignment, and small stacks: one thread per packed word.
 template <int OUT>  // 0 bf16, 1 fp16, 2 fp32
 __global__ __launch_bounds__(256) void dequant_kernel(ProjDev p, const int32_t* __restrict__ g_idx,
                                                       int K, int N, int G, int linear,
@@ -195,15 +195,40 @@ __global__ __launch_bounds__(256) void dequant_kernel(ProjDev p, const int32_t* 
   }
 }
 
+// Whether the tile kernel is the faster one, from both kernels' times over 2^14 to 2^22 packed words
+// of 8 to 2048 k and 8 to 2048 columns (in ps beyond a launch of 3.4 us). The one-thread-per-word
+// kernel takes 10 per word (7 in long rows of words) and 3 per thread, and 256 threads cover a
+// row's columns. The tile kernel takes a fixed chain of loads, LDS and stores, plus a share per tile
+// of 32 packed rows x 64 columns, full or not, and with g_idx of the tile's table. bf16 linear: 1 expert of 512 x 512 3.7 against 6.1 us, 2 of 2048 x 512
+// 8.0 against 6.8, 4 of them 11.1 against 7.4, 256 of 24 x 512 8.7 against 16.0.
+bool tile_pays(int64_t E, int64_t K, int64_t N, int64_t G, bool linear, bool fp32, bool idx) {
+  const int64_t words = E * (K / 8) * N, threads = E * (K / 8) * ((N + 255) / 256 * 256);
+  const int64_t tiles = E * ((K / 8 + kTileR - 1) / kTileR) * ((N + kTileC - 1) / kTileC);
+  int64_t base, per_tile;
+  if (linear) {
+    base = fp32 ? 1400000 : 2600000;
+    per_tile = fp32 ? 2700 : 4900;
+  } else if (fp32) {
+    base = idx ? 3300000 : 1300000;
+    per_tile = 500;
+  } else {  // stores of 8 bytes: partial lines where the columns end inside a tile
+    base = idx ? 8000000 : (N % kTileC ? 6000000 : 2200000);
+    per_tile = 2000;
+  }
+  if (idx) per_tile += 160 * (K / G);
+  return (N >= 1024 ? 7 : 10) * words + 3 * threads > base + per_tile * tiles;
+}
+
 template <int OUT>
 hipError_t launch_out(const ProjDev& p, const int32_t* g_idx, int E, int K, int N, int G,
                       int linear, void* out, hipStream_t stream) {
   const uintptr_t bases = reinterpret_cast<uintptr_t>(p.qweight) |
                           reinterpret_cast<uintptr_t>(p.scales) | reinterpret_cast<uintptr_t>(out);
-  // The tile kernel (117.5 -> 39 us a call, see there) wherever its accesses fit: its loads and
-  // stores are up to 16 bytes wide, its words lie in one group
-  // (without g_idx) and its group table (with g_idx) holds kMaxIdxGroups.
-  const bool tile = (bases & 15u) == 0 && (g_idx ? K / G <= kMaxIdxGroups : G % 8 == 0);
+  // The tile kernel where its accesses fit (its loads and stores are up to 16 bytes wide, its
+  // words lie in one group (without g_idx) and its group table (with g_idx) holds
+  // kMaxIdxGroups) and where it pays.
+  const bool tile = (bases & 15u) == 0 && (g_idx ? K / G <= kMaxIdxGroups : G % 8 == 0) &&
+                    tile_pays(E, K, N, G, linear != 0, OUT == 2, g_idx != nullptr);
   if (!tile) {
     hipLaunchKernelGGL(dequant_kernel<OUT>, dim3((N + 255) / 256, K / 8, E), dim3(256), 0, stream,
                        p, g_idx, K, N, G, linear, out);

@@ -34,8 +34,11 @@ def test_dequant_bit_exact(E, K, N, linear):
 
 # (E, K, N, G): one row past a tile of 32 packed rows and 8 columns past one of 64; the smallest;
 # the most groups the tile's table holds (64) and more; a group that a packed word straddles
+# The large stacks take the tile kernel, the small ones the one for small stacks.
 @pytest.mark.parametrize("E,K,N,G", [(2, 264, 72, 24), (3, 8, 8, 8), (1, 512, 136, 8),
-                                     (1, 1024, 64, 8), (2, 24, 16, 12)])
+                                     (1, 1024, 64, 8), (2, 24, 16, 12),
+                                     (400, 264, 72, 24), (4000, 8, 8, 8), (100, 512, 136, 8),
+                                     (100, 1024, 64, 8), (2000, 24, 16, 12)])
 @pytest.mark.parametrize("linear", [True, False])
 @pytest.mark.parametrize("act_order", [False, True])
 @pytest.mark.parametrize("offset", [0, 1])
@@ -66,6 +69,27 @@ def test_dequant_tile_edges(E, K, N, G, linear, act_order, offset):
         got = ops.dequantize(dev(q), dev(z), dev(s), dev(gi.int()) if act_order else None,
                              group_size=G, linear_weight=linear, dtype=dtype).cpu()
         assert torch.equal(got, want.to(dtype)), dtype
+
+
+# (E, K, N, G): small stacks; a few packed rows, which leave a tile mostly empty; a large stack
+@pytest.mark.parametrize("E,K,N,G,most", [(1, 512, 512, 64, 1.25), (64, 40, 72, 8, 1.25),
+                                          (256, 24, 512, 24, 1.25), (32, 2048, 512, 128, 0.7)])
+def test_dequant_costs_no_more_than_a_thread_per_word(E, K, N, G, most):
+    """A base that is not 16-byte aligned always takes one thread per packed word: an aligned call
+    costs no more (the margin is for noise; 1.6 times as much where small stacks took the tiles),
+    and for a large stack a good deal less (0.33 measured)."""
+    from tests.helpers import graph_us
+    us = []
+    for offset in (0, 1):
+        def dev(shape, dtype):
+            n = int(np.prod(shape))
+            flat = torch.randint(0, 2**15, (n + offset,), device="cuda").to(dtype)
+            return flat[offset:].view(shape)
+        q, z = dev((E, K // 8, N), torch.int32), dev((E, K // G, N // 8), torch.int32)
+        s = dev((E, K // G, N), torch.float16)
+        us.append(graph_us(lambda: ops.dequantize(q, z, s, group_size=G)))
+    _say(f"dequant E={E} K={K} N={N}: aligned {us[0]:.2f} us, not aligned {us[1]:.2f} us")
+    assert us[0] < most * us[1]
 
 
 def test_dequant_reference_kat_and_g_idx():
