@@ -18,20 +18,20 @@ namespace {
 MOE_DEV uint16_t silu_bf16(float v) { return (uint16_t)f32_to_bf16_rne(v / (1.0f + expf(-v))); }
 
 // x[head][t][:] . W[head][n][:] for the 4 waves x TE rows n of a workgroup, head = blockIdx.y, and
-// the token tiles of its kTokensPerWg tokens: every wave issues the loads of its
+// the token tiles of its per_wg tokens: every wave issues the loads of its
 // weight rows, then each tile of TT token rows passes through LDS, so a weight row is read once
-// for kTokensPerWg tokens and the whole 8 KB of a wave's rows is in flight at once (bound by HBM up
+// for per_wg tokens and the whole 8 KB of a wave's rows is in flight at once (bound by HBM up
 // to about 4 tokens, by the fp32 FMAs beyond). 40 heads (2048 -> 1024 -> 256, 189 MB) per call:
 // 4 tokens 116.7 -> 50.6 us (the row read from memory once per token before), 1 token 37.5 us, 16
 // tokens 89 us. Two rows per wave (four: 58.3 us at 4 tokens, one: 57.4) and nontemporal
 // weight loads (53.5 -> 50.6).
 // ACT: out is bf16 [n / D][T][D] = silu(z); else fp32 [head][T][N + 1].
-constexpr int kRowsTE = 2, kTokensPerWg = 32;
+constexpr int kRowsTE = 2;
 template <int TT, int NI, bool ACT>
 __global__ __launch_bounds__(256) void mlp_rows_kernel(const uint16_t* __restrict__ x,
                                                        int64_t x_head, int T, int K,
                                                        const uint16_t* __restrict__ W,
-                                                       int64_t w_head, int N, int D,
+                                                       int64_t w_head, int N, int D, int per_wg,
                                                        void* __restrict__ out_v) {
   __shared__ __attribute__((aligned(16))) uint16_t s_x[TT * NI * 512];
   constexpr int NV = TT * kRowsTE;
@@ -43,8 +43,8 @@ __global__ __launch_bounds__(256) void mlp_rows_kernel(const uint16_t* __restric
   LdsLogitsTile<TT, kRowsTE, NI, kBufNontemporal> tile;
   tile.load(K, W + head * w_head, N, nullptr, n0, lane);
   const __amdgpu_buffer_rsrc_t xr = buf_rsrc(x + head * x_head, (uint32_t)T * (uint32_t)K * 2u);
-  const int t_begin = (int)blockIdx.x / row_blocks * kTokensPerWg;
-  const int t_end = min(T, t_begin + kTokensPerWg);
+  const int t_begin = (int)blockIdx.x / row_blocks * per_wg;
+  const int t_end = min(T, t_begin + per_wg);
   for (int t0 = t_begin; t0 < t_end; t0 += TT) {
     if (t0 > t_begin) __syncthreads();  // the previous tile is read
     // the tile's rows are contiguous; past the last token the loads read zeros
@@ -121,15 +121,25 @@ hipError_t launch_mlp_logits(const uint16_t* x, int64_t x_head, int T, int K, co
 
 // The tiled products hold K in at most four 512-column steps per lane.
 constexpr int kRowsMaxK = 2048;
+constexpr int kMaxTokensPerWg = 32, kWantedWgs = 1024;
 
 template <int NI, bool ACT>
 hipError_t launch_mlp_rows(const uint16_t* x, int64_t x_head, int T, int K, const uint16_t* W,
                            int64_t w_head, int N, int D, void* out, int heads,
                            hipStream_t stream) {
   const unsigned row_blocks = (N + 4 * kRowsTE - 1) / (4 * kRowsTE);
-  const dim3 grid(row_blocks * ((T + kTokensPerWg - 1) / kTokensPerWg), heads);
+  // Tokens per workgroup: its token tiles run one after the other, so with few rows they are dealt to
+  // more workgroups, down to one tile each, until there are four per CU (the weight rows then come
+  // from L2 again). One head (2048 -> 1024 -> 256): 32 tokens 31.7 us at 32 per workgroup, 13.8 so;
+  // 8 heads 43.9 -> 38.2. Wanting 512 is slower (40 heads of 512, 32 tokens 52.7 against 51.0 us),
+  // 2048 reads the weights too often (8 heads, 8 tokens 22.4 against 19.4).
+  int per_wg = kMaxTokensPerWg;
+  while (per_wg > 4 && (int64_t)row_blocks * heads * ((T + per_wg - 1) / per_wg) < kWantedWgs)
+    per_wg /= 2;
+  const dim3 grid(row_blocks * ((T + per_wg - 1) / per_wg), heads);
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, x_head, T, K, W, w_head, N, D, out);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, x, x_head, T, K, W, w_head, N, D, per_wg,
+                       out);
     return hipGetLastError();
   };
   // the token tile nearest to the batch: rows of a larger one would be zeros. 4 tokens at most:
