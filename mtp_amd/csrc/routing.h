@@ -470,15 +470,17 @@ MOE_DEV uint64_t expert_peers(int e) {
 }
 
 // topk_ids in global memory. One workgroup, so what bounds it is its chain of dependent steps.
-// Up to kAlignIds chunks of 64 slots per wave (8192 slots) a wave's ids stay in registers from the
+// Up to kAlignHeld chunks of 64 slots per wave (4096 slots) a wave's ids stay in registers from the
 // one load on: the ballot match ranks a chunk's slots and leaves the wave's counts behind, one
 // pass over the groups turns the counts into bases, and the slots, the padding and the block ids
 // are stored together after the last barrier (a barrier between stores waits for the earlier
 // ones). Against counting with LDS atomics, loading the ids a second time and ranking them after
 // the padding's stores: eight layers of 48 tokens (64 experts, top-4) 168.5 -> 163.5 us, of 64
 // tokens (256 experts, top-8) 524 -> 514 us; one layer of 203 tokens 98.7 -> 97.7 us. Larger
-// inputs keep that form: their ids do not fit the registers.
+// inputs keep that form: their slots' stores are better spread between the ranks (8192 slots of 512
+// experts 13.2 against 15.0 us held, 5000 10.7 against 11.3, 3000 9.1 against 9.0).
 // With fill_tail false the entries past the padded total are left as they are, as in align_wave.
+constexpr int kAlignHeld = 4;
 MOE_DEV void align_block(const int32_t* topk_ids, int T, int top_k, int E, int has_shared, int BM,
                          int cap, int32_t* __restrict__ sorted, int32_t* __restrict__ eids,
                          int32_t* __restrict__ ntpp, AlignSmem& sm, bool fill_tail) {
@@ -489,17 +491,17 @@ MOE_DEV void align_block(const int32_t* topk_ids, int T, int top_k, int E, int h
   const BlockDiv bd(BM);
   const int per_wave = (((n_slots + kAlignWaves - 1) / kAlignWaves) + 63) / 64 * 64;
   const int lo = min(w * per_wave, n_slots), hi = min(lo + per_wave, n_slots);
-  const bool held = per_wave <= 64 * kAlignIds;  // uniform over the workgroup
+  const bool held = per_wave <= 64 * kAlignHeld;  // uniform over the workgroup
   const __amdgpu_buffer_rsrc_t ir = buf_rsrc(topk_ids, (uint32_t)routed * 4u);
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  int eb[kAlignIds], rank[kAlignIds];
-  align_ids(ir, routed, E, lo, hi, lane, eb);
+  int eb[kAlignIds], rank[kAlignHeld];
+  if (held) align_ids(ir, routed, E, lo, hi, lane, eb);
   // every wave clears and fills its own counters: LDS operations of one wave complete in order
   for (int g = lane; g < G; g += 64) sm.cnt[w][g] = 0;
   __builtin_amdgcn_wave_barrier();
   if (held) {
 #pragma unroll
-    for (int u = 0; u < kAlignIds; ++u) {
+    for (int u = 0; u < kAlignHeld; ++u) {
       if (lo + 64 * u >= hi) break;  // uniform over the wave
       const int e = eb[u];
       const uint64_t peers = expert_peers(e);
@@ -548,7 +550,7 @@ MOE_DEV void align_block(const int32_t* topk_ids, int T, int top_k, int E, int h
   // Stable scatter: ranges in wave order, slots in order inside a range.
   if (held) {
 #pragma unroll
-    for (int u = 0; u < kAlignIds; ++u) {
+    for (int u = 0; u < kAlignHeld; ++u) {
       if (lo + 64 * u >= hi) break;  // uniform over the wave
       if (eb[u] >= 0) {
         const int pos = sm.cnt[w][eb[u]] + rank[u];

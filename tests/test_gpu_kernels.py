@@ -192,8 +192,9 @@ def test_align_bit_exact(T, k, E, BM, shared, zipf):
 
 @pytest.mark.parametrize("T,k,E,BM,shared", [(65, 1, 512, 16, True),  # a second chunk, 513 groups
                                              (203, 8, 256, 16, True),
-                                             # 8192 slots: the last that the registers hold; then
-                                             # one more token
+                                             # 4096 slots: the last that the registers hold; then
+                                             # one more token; the same of the ids that one load takes
+                                             (512, 8, 64, 16, False), (513, 8, 64, 16, False),
                                              (1024, 8, 64, 16, False), (1025, 8, 64, 16, False)])
 def test_align_held_ids(T, k, E, BM, shared):
     """The one-workgroup align with several chunks per wave, with experts that fill whole chunks
