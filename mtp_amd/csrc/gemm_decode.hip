@@ -669,6 +669,11 @@ hipError_t launch_decode_cfg(const uint16_t* act, const ExpertsDev& ed, const Sl
 //    these some CUs would get one such workgroup and others two (8 tokens: 267 against 257), and
 //    below there are too few. The workgroups are estimated from the experts that an even routing
 //    reaches. K of 512 is too short to gain from it (64 tokens: 239 against 234 us).
+//  - Where an expert has 8 rows and more, blocks are full and experts have several: four columns
+//    from 500 workgroups on, at K of 512 too (a layer of hidden 2048, intermediate 512: 1200
+//    tokens, top-2, 16 experts 71.1 against 81.3 us, 128 tokens, top-8, 64 experts 58.5 against
+//    62.2; hidden 512: 256 tokens, top-8, 64 experts 48.9 against 53.0). Not with two waves (6
+//    groups of 256), whose four-column form has one wave per SIMD: 46.9 against 50.6 there.
 //  - Up to 16 slots W1 takes eight waves: nothing but latency counts there.
 template <int MODE>
 DecodeCfg pick_decode_cfg(const ExpertsDev& ed, const SlotsDev& sd) {
@@ -680,6 +685,9 @@ DecodeCfg pick_decode_cfg(const ExpertsDev& ed, const SlotsDev& sd) {
     const float reached = E * (1.0f - powf(fmaxf(0.0f, 1.0f - (float)sd.top_k / E), (float)sd.T));
     const float wgs = reached * (float)(ed.inter / 64);
     if (K <= 512 || wgs < 220.0f || (wgs > 300.0f && wgs < 700.0f)) c.ct = 2;
+    const float slots = (float)sd.T * (float)sd.top_k;
+    const float blocks = fmaxf(reached, slots / 16.0f + reached / 2.0f);
+    if (c.ks == 4 && slots >= 8.0f * reached && blocks * (float)(ed.inter / 64) >= 500.0f) c.ct = 4;
     if (sd.num_slots <= 16 && groups % 8 == 0) c = DecodeCfg{8, 2};
   }
   return c;

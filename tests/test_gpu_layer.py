@@ -99,12 +99,21 @@ def test_decode_shapes_and_groups(E, H, I, G, shared, T):
 def test_decode_tiles(H, G):
     """Every tile of the decode GEMMs (waves over K, groups per wave, columns per lane): 12 tokens
     take two columns per lane in W1 at intermediate 256 and 512 and, from hidden 1024 on, four at
-    1024 (about 250 workgroups); 2 tokens eight waves over K where the groups allow it, 5 the
-    token-sum W2 of each intermediate size."""
-    for I, T in ((256, 12), (512, 12), (1024, 12), (512, 2), (256, 5), (512, 5), (1024, 5)):
+    1024 (about 250 workgroups); 3 tokens (2 take the fused kernel at group 128) eight waves over K
+    where the groups allow it, 5 the token-sum W2 of each intermediate size."""
+    for I, T in ((256, 12), (512, 12), (1024, 12), (512, 2), (512, 3), (256, 5), (512, 5), (1024, 5)):
         _say(f"decode tiles H={H} G={G} I={I} T={T}")
         layer = synth.make_layer(4, num_experts=16, hidden=H, intermediate=I, group=G)
         _check_layer(layer, T, 4, "decode")
+
+
+@pytest.mark.parametrize("H", [512, 2048])
+@pytest.mark.parametrize("G", [64, 128])
+def test_decode_tiles_of_many_rows_per_expert(H, G):
+    """Four columns per lane where every expert has several full blocks, at hidden 512 too."""
+    _say(f"decode tiles of full blocks H={H} G={G}")
+    layer = synth.make_layer(4, num_experts=8, hidden=H, intermediate=512, group=G)
+    _check_layer(layer, 250, 4, "decode")
 
 
 @pytest.mark.parametrize("T", [1, 32])
