@@ -261,6 +261,7 @@ int64_t moe_predictor_workspace_bytes_v1(int32_t T, int32_t num_heads, int32_t i
                                          int32_t num_experts, int32_t top_k) {
   if (T < 0 || num_heads < 1 || inner < 1 || num_experts < 1 || top_k < 1) return -1;
   const size_t L = num_heads;
+  // z1 (the first section) is written for hidden beyond 2048 only, which the query does not know
   return (int64_t)(align256((size_t)T * (L * inner + 1) * 4) + align256(L * T * inner * 2) +
                    align256(L * T * (num_experts + 1) * 4) + align256(L * T * top_k * 4));
 }

@@ -88,11 +88,6 @@ struct GroupSZ {
   uint32_t s[NP][CT / 2];       // fp16 scale pairs of the CT columns
   uint32_t z[NP];               // packed zeros word holding the CT columns
 };
-template <int NP, int SPG, int CT>
-struct GroupBuf {
-  GroupAW<NP, SPG, CT> aw;
-  GroupSZ<NP, CT> sz;
-};
 
 // A operand of one lane: resource over the activation rows and the byte offset of
 // (this lane's row, first k of the wave's slice + 8 * kq), kOutOfRange for a padding row.
@@ -173,16 +168,7 @@ struct DecodeTile {
     }
   }
 
-  MOE_DEV void load(GroupBuf<NP, SPG, CT>& B, int gi) const {
-    load_aw(B.aw, gi);
-    load_sz(B.sz, gi);
-  }
-
-  // acc[p*CT + j] += s * (sum_k x (128 + q) - (128 + z) * sum_k x) over one group. A group
-  // past the slice loaded zeros (scale 0) and adds +0.
-  MOE_DEV void compute(const GroupBuf<NP, SPG, CT>& B, f32x4 (&acc)[NP * CT]) const {
-    compute(B.aw, B.sz, acc);
-  }
+  // acc[p*CT + j] += s * (sum_k x (128 + q) - (128 + z) * sum_k x) over one group.
   MOE_DEV void compute(const GroupAW<NP, SPG, CT>& B, const GroupSZ<NP, CT>& Z,
                        f32x4 (&acc)[NP * CT]) const {
     const bf16x8_v ones = as_frag(kOnes, kOnes, kOnes, kOnes);
@@ -639,7 +625,7 @@ hipError_t launch_decode_cfg(const uint16_t* act, const ExpertsDev& ed, const Sl
   if constexpr (MODE == DEC_W1) {
     if constexpr (SPG == 2) { MOE_DEC2(4, 2) MOE_DEC2(4, 4) MOE_DEC2(4, 6) MOE_DEC2(4, 8) }
     if constexpr (SPG == 4) { MOE_DEC2(4, 1) MOE_DEC2(4, 2) MOE_DEC2(4, 3) MOE_DEC2(4, 4) }
-    if constexpr (SPG == 8) { MOE_DEC2(4, 1) MOE_DEC2(4, 2) MOE_DEC2(2, 1) MOE_DEC2(2, 3) }
+    if constexpr (SPG == 8) { MOE_DEC2(4, 1) MOE_DEC2(4, 2) MOE_DEC(2, 2, 1) MOE_DEC2(2, 3) }
     MOE_DEC(8, 2, 1)
     if constexpr (SPG <= 4) { MOE_DEC(8, 2, 2) }
     if constexpr (SPG == 2) { MOE_DEC(8, 2, 3) MOE_DEC(8, 2, 4) }

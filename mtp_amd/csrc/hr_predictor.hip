@@ -402,7 +402,8 @@ int hr_check(int32_t N, const moe_hr_predictor_params_v1* p, int32_t top_k) {
       top_k > 64)
     return hr_fail(MOE_ERR_SHAPE, "num_experts in [1, 512] and top_k in [1, min(E, 64)]");
   if (!(p->ln_eps >= 0.0f)) return hr_fail(MOE_ERR_SHAPE, "ln_eps must be >= 0");
-  // 32-bit offsets of the buffers and of the workspace's sections
+  // 32-bit offsets of the buffers and of the four-launch form's sections (asked of either form, so
+  // that what is refused does not depend on which one a size takes)
   const int64_t lim = int64_t(1) << 31;
   if ((int64_t)N * p->hidden * 2 >= lim || (int64_t)p->width * p->hidden * 2 >= lim ||
       (int64_t)N * p->future_window * p->width * 2 >= lim ||
