@@ -546,6 +546,39 @@ def test_prefill_router_certificate_on_ties(shared):
         assert moe_ref.rel_err(out.float().cpu().numpy(), ref) <= LAYER_RTOL
 
 
+@pytest.mark.parametrize("top_k", [8, 13, 64])  # 13: a batch of canonical dots and a rest of odd size
+@pytest.mark.parametrize("T,E", [(200, 512), (1061, 512)])  # 32 x 64 and 64 x 64 tiles
+def test_prefill_router_certificate_on_near_ties(T, E, top_k):
+    """Router rows that differ from one another in the last bit of 0 to 95 elements: the logits of a
+    token's selection and of the experts behind it lie from nothing to many times the error bound
+    apart, so some tokens are certified and others recompute candidates. Ids and weights are the
+    canonical router's bit for bit."""
+    H, rows = 1024, 96
+    _say(f"prefill router near-ties T={T} E={E} top_k={top_k}")
+    layer = to_gpu(synth.make_layer(7, num_experts=E, hidden=H, intermediate=256, shared=True))
+    g = torch.Generator().manual_seed(79)
+    v = (torch.randn(H, generator=g) * 0.08).to(torch.bfloat16)
+    rw = layer.router_w.cpu().clone()
+    for j, e in enumerate(torch.randperm(E, generator=g)[:rows].tolist()):
+        at = torch.randperm(H, generator=g)[:j]
+        bits = v.view(torch.int16).clone()
+        bits[at] ^= 1
+        rw[e] = bits.view(torch.bfloat16)
+    rw = rw.cuda()
+    x = synth.make_tokens(T, H, seed=80).cuda()
+    x[::2] = (x[::2].float() + 4 * v.cuda().float()).to(torch.bfloat16)  # these select the near rows
+    _, ids, w = ops.moe_layer(x, rw, layer.experts, top_k=top_k, shared=layer.shared,
+                              shared_gate_w=layer.shared_gate_w, path="prefill",
+                              return_routing=True)
+    r_ids, r_w, _, logits = ops.router_topk(x, rw, top_k, shared_gate_w=layer.shared_gate_w)
+    top = logits.topk(top_k + 1, dim=1).values
+    gap = (top[:, top_k - 1] - top[:, top_k]).cpu()
+    _say(f"  gaps at the selection's edge: {int((gap < 1e-5).sum())} below 1e-5, "
+         f"{int((gap < 1e-3).sum())} below 1e-3 of {T}")
+    assert (gap < 1e-3).sum() > T // 20 and (gap > 1e-2).sum() > T // 20
+    assert torch.equal(ids, r_ids) and torch.equal(w, r_w)
+
+
 @pytest.mark.parametrize("T,path,top_k", [(3, "decode", 8), (3, "decode", 16), (40, "decode", 8),
                                           (9, "decode", 16), (300, "prefill", 8),
                                           (1100, "prefill", 8)])
