@@ -15,13 +15,13 @@
 // exact products in fp32, on v_mfma_f32_16x16x32_bf16 or in the router's canonical order
 // (routing.h:logits_tile). At these sizes a call is bound by launches and by each kernel's chain
 // of loads, not by bytes or arithmetic. Two forms (hr_split chooses):
-//  - two launches: the encoder, then everything per 16 context rows (hr_rows_kernel). Each of its
-//    workgroups reads the whole classifier, so it is the form for many rows or a small classifier:
-//    160 examples of the default shape (hidden 2048, width 256, 4 deltas, 256 experts, top-16)
-//    21.4 us, in the other form with the canonical encoder 53.5;
-//  - four launches for few rows of a large classifier: the encoder, the context rows, the
-//    classifier over many workgroups, the selection: one example and delta of width 256 13.6 us
-//    (17.2 in the other form), of width 512 14.4 (25.8), of width 1024 and 512 experts 20 (55).
+//  - two launches: the encoder, then everything per 16 context rows (hr_rows_kernel): 160 examples
+//    of the default shape (hidden 2048, width 256, 4 deltas, 256 experts, top-16) 19 us on the GPU
+//    and 22 us a call, which the host's work bounds (four launches: 29 to 53 us);
+//  - four launches for few rows of a large classifier, which one workgroup of the first form would
+//    read alone: the encoder, the context rows, the classifier over many workgroups, the
+//    selection: one example and delta of width 1024 with 512 experts 20.8 us on the GPU and 29 a
+//    call (46 and 46 in two launches).
 // The error against 64 bits is the same (3.7e-3 to 4.2e-3 of the residual over 3 to 640 examples
 // and widths 128 to 512: the bf16 activations).
 #include <math.h>
@@ -96,18 +96,25 @@ __global__ __launch_bounds__(64 * kEncWaves) void hr_encoder_kernel(
 // (wave w the expert tiles w, w + 16); then v = (prior ? prior[r] : 0) + scale_n * logits[r],
 // optionally written to out, and the top-k of v by (value, lower id), again one wave per row, so
 // that the 16 selections of a workgroup run side by side (each is a serial chain of top_k rounds).
-// The classifier rows of the first 256 k and the row's prior are loaded before anything else. NC,
-// MAXC: 64-lane columns of the width and of the experts. The F rows of one example repeat its
-// LayerNorm: cheaper than another launch.
-constexpr int kRows = 16, kClsSteps = 8;
+// What bounds it is the memory round trips of that chain, so every operand of the context row, the
+// prior, the bias and the first classifier steps are loaded together, four columns a lane (one
+// column a lane with the loads behind their range checks: one example 12.4 us against 10.6 at
+// width 256, 20.3 against 14.2 at width 512), and a wave keeps kRing classifier steps in flight.
+// NC, MAXC: 64-lane columns of the width and of the experts. The F rows of one example repeat its
+// LayerNorm: cheaper than another launch. 64 VGPRs where that fits: two workgroups per CU (5120
+// rows of width 128: 33.5 us, with one 36.7).
+constexpr int kRows = 16;
 template <int NC, int MAXC>
-__global__ __launch_bounds__(64 * kRows) void hr_rows_kernel(
+__global__ __launch_bounds__(64 * kRows, NC + MAXC == 8 ? 8 : 4) void hr_rows_kernel(
     const float* __restrict__ z, int rows, int F, const int32_t* __restrict__ layer_ids,
     moe_hr_predictor_params_v1 p, const float* __restrict__ prior, float scale,
     const float* __restrict__ scale_per_example, int top_k, float* __restrict__ out,
     int32_t* __restrict__ ids) {
   constexpr int kG = 64 * NC + 8, kL = 64 * MAXC + 4;  // row strides (16-byte rows, odd quads)
   constexpr int TPW = MAXC / 4;                        // expert tiles per wave
+  constexpr int NQ = NC / 4;                           // column quads per lane
+  // classifier k-steps of 32: in all, in the ring of a wave, and of these loaded before the context
+  constexpr int kSteps = 2 * NC, kRing = 16 / TPW < kSteps ? 16 / TPW : kSteps, kFirst = 8 / TPW;
   __shared__ __attribute__((aligned(16))) uint16_t s_g[kRows * kG];
   __shared__ float s_l[kRows * kL];
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
@@ -116,81 +123,117 @@ __global__ __launch_bounds__(64 * kRows) void hr_rows_kernel(
   const int row = (int)blockIdx.x * kRows + wv;
   const bool live = row < rows;  // wave-uniform
   const int n = live ? row / F : 0, d = live ? row % F : 0;
+  const int layer = layer_ids[n];
+  const bool layer_ok = layer >= 0 && layer < p.num_layers;  // else the embedding reads zeros
+  const float sc = scale_per_example ? scale_per_example[n] : scale;
 
-  const __amdgpu_buffer_rsrc_t cr = buf_rsrc(p.cls_w, (uint32_t)E * (uint32_t)W * 2u);
-  u32x4 b[TPW][kClsSteps];
-  auto load_cls = [&](int k0) {
+  // The context row's operands (lane: columns 4 (lane + 64 i) ..; past the width zeros, without a
+  // memory access), the prior, the classifier's bias and its first chunk: one memory latency.
+  const uint32_t wb = (uint32_t)W * 2u;
+  const __amdgpu_buffer_rsrc_t zr = buf_rsrc(z + (int64_t)n * (W + 1), 2u * wb);
+  const __amdgpu_buffer_rsrc_t br = buf_rsrc(p.enc_b, 2u * wb);
+  const __amdgpu_buffer_rsrc_t lwr = buf_rsrc(p.ln_w, wb), lbr = buf_rsrc(p.ln_b, wb);
+  const __amdgpu_buffer_rsrc_t ler =
+      buf_rsrc(p.layer_emb + (int64_t)(layer_ok ? layer : 0) * W, layer_ok ? wb : 0u);
+  const __amdgpu_buffer_rsrc_t der = buf_rsrc(p.delta_emb + (int64_t)d * W, wb);
+  u32x4 zq[NQ], bq[NQ];
+  u32x2 lw[NQ], lb[NQ], le[NQ], de[NQ];
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const int e = 16 * (wv + 16 * t) + r16;
-      const uint32_t eo = e < E ? (uint32_t)e * (uint32_t)W * 2u : kOutOfRange;
-#pragma unroll
-      for (int i = 0; i < kClsSteps; ++i) {
-        const int k = k0 + 32 * i + 8 * kq;
-        const uint32_t ko = k < W ? (uint32_t)k * 2u : kOutOfRange;
-        b[t][i] = buf_ld128(cr, (eo + ko) | ((eo | ko) & kOutOfRange));
-      }
-    }
-  };
-  load_cls(0);
+  for (int i = 0; i < NQ; ++i) {
+    const uint32_t q = (uint32_t)(lane + 64 * i);
+    zq[i] = buf_ld128(zr, q * 16u);
+    bq[i] = buf_ld128(br, q * 16u);
+    lw[i] = buf_ld64(lwr, q * 8u);
+    lb[i] = buf_ld64(lbr, q * 8u);
+    le[i] = buf_ld64(ler, q * 8u);
+    de[i] = buf_ld64(der, q * 8u);
+  }
   const __amdgpu_buffer_rsrc_t pr = buf_rsrc(prior ? prior + (int64_t)(live ? row : 0) * E : nullptr,
                                              prior && live ? (uint32_t)E * 4u : 0u);
-  float pv[MAXC];
+  float pv[MAXC], cb[TPW];
 #pragma unroll
   for (int c = 0; c < MAXC; ++c)
     pv[c] = __uint_as_float(buf_ld32(pr, (uint32_t)(lane + 64 * c) * 4u));
-
-  // context row (lane: columns lane + 64 i); columns past the width hold zeros
-  float a[NC], sum = 0.0f;
-  const __amdgpu_buffer_rsrc_t zr = buf_rsrc(z + (int64_t)n * (W + 1), (uint32_t)W * 4u);
+  const __amdgpu_buffer_rsrc_t cbr = buf_rsrc(p.cls_b, (uint32_t)E * 4u);
 #pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const int j = lane + 64 * i;
-    const float zb = bf16_round(__uint_as_float(buf_ld32(zr, (uint32_t)j * 4u)) +
-                                (j < W ? p.enc_b[j] : 0.0f));
-    a[i] = j < W ? bf16_round(zb / (1.0f + expf(-zb))) : 0.0f;
-    sum += a[i];
-  }
+  for (int t = 0; t < TPW; ++t)
+    cb[t] = __uint_as_float(buf_ld32(cbr, (uint32_t)(16 * (wv + 16 * t) + r16) * 4u));
+  const __amdgpu_buffer_rsrc_t cr = buf_rsrc(p.cls_w, (uint32_t)E * wb);
+  u32x4 b[kRing][TPW];
+  auto load_cls = [&](int i) {  // k-step i into its place in the ring
+    const int k = 32 * i + 8 * kq;
+    const uint32_t ko = k < W ? (uint32_t)k * 2u : kOutOfRange;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      const int e = 16 * (wv + 16 * t) + r16;
+      const uint32_t eo = e < E ? (uint32_t)e * wb : kOutOfRange;
+      b[i % kRing][t] = buf_ld128(cr, (eo + ko) | ((eo | ko) & kOutOfRange));
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < kFirst; ++i) load_cls(i);
+  __builtin_amdgcn_sched_barrier(0);
+
+  float a[4 * NQ], sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NQ; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float zb = bf16_round(__uint_as_float(zq[i][j]) + __uint_as_float(bq[i][j]));
+      // a column past the width has z = bias = 0 and silu(0) = 0
+      a[4 * i + j] = bf16_round(zb / (1.0f + expf(-zb)));
+      sum += a[4 * i + j];
+    }
   const float mean = bfly_sum(sum) / (float)W;
   float sq = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const float dv = lane + 64 * i < W ? a[i] - mean : 0.0f;
-    sq = __builtin_fmaf(dv, dv, sq);
-  }
+  for (int i = 0; i < NQ; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float dv = 4 * (lane + 64 * i) < W ? a[4 * i + j] - mean : 0.0f;
+      sq = __builtin_fmaf(dv, dv, sq);
+    }
   const float var = bfly_sum(sq) / (float)W;
   const float rstd = 1.0f / sqrtf(var + p.ln_eps);
-  const int layer = layer_ids[n];
-  const bool layer_ok = layer >= 0 && layer < p.num_layers;  // else the embedding reads zeros
+  auto el = [](u32x2 v, int j) { return (j & 1) ? bf16hi_to_f32(v[j >> 1]) : bf16lo_to_f32(v[j >> 1]); };
 #pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const int j = lane + 64 * i;
-    uint16_t g = 0;
-    if (j < W) {
-      const float s =
-          bf16_round((a[i] - mean) * rstd * bf16_to_f32(p.ln_w[j]) + bf16_to_f32(p.ln_b[j]));
-      const float le = layer_ok ? bf16_to_f32(p.layer_emb[(int64_t)layer * W + j]) : 0.0f;
-      const float sl = bf16_round(s + le);
-      const float c = bf16_round(sl + bf16_to_f32(p.delta_emb[(int64_t)d * W + j]));
-      g = (uint16_t)f32_to_bf16_rne(c / (1.0f + expf(-c)));
+  for (int i = 0; i < NQ; ++i) {
+    const uint32_t in = 0u - (uint32_t)(4 * (lane + 64 * i) < W);
+    uint32_t g[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float s = bf16_round((a[4 * i + j] - mean) * rstd * el(lw[i], j) + el(lb[i], j));
+      const float sl = bf16_round(s + el(le[i], j));
+      const float c = bf16_round(sl + el(de[i], j));
+      g[j] = f32_to_bf16_rne(c / (1.0f + expf(-c))) & in;
     }
-    s_g[wv * kG + j] = g;
+    *reinterpret_cast<u32x2*>(s_g + wv * kG + 4 * (lane + 64 * i)) =
+        u32x2{g[0] | (g[1] << 16), g[2] | (g[3] << 16)};
   }
-  __syncthreads();
+#pragma unroll
+  for (int i = kFirst; i < kRing; ++i) load_cls(i);
+  // A barrier without __syncthreads' fence, which would also wait for the loads in flight.
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
 
-  // classifier: A row r16 at k = 32 step + 8 kq from LDS, B from the loaded rows
+  // classifier: A row r16 at k = 32 step + 8 kq from LDS
   f32x4 acc[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < W; k0 += 32 * kClsSteps) {
-    if (k0 > 0) load_cls(k0);
 #pragma unroll
-    for (int i = 0; i < kClsSteps; ++i) {
-      const int k = k0 + 32 * i;
-      if (k >= 64 * NC) break;
-      const u32x4 av = ld128(s_g + r16 * kG + k + 8 * kq);
+  for (int i0 = 0; i0 < kSteps; i0 += 4) {
+    u32x4 av[4];
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) acc[t] = mfma16(av, b[t][i], acc[t]);
+    for (int i = 0; i < 4; ++i) av[i] = ld128(s_g + r16 * kG + 32 * (i0 + i) + 8 * kq);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) acc[t] = mfma16(av[i], b[(i0 + i) % kRing][t], acc[t]);
+    if (i0 + kRing < kSteps) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) load_cls(i0 + i + kRing);
+      __builtin_amdgcn_sched_barrier(0);  // the ring's loads here, not at their use
     }
   }
 #pragma unroll
@@ -198,12 +241,11 @@ __global__ __launch_bounds__(64 * kRows) void hr_rows_kernel(
     const int e = 16 * (wv + 16 * t) + r16;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (e < E) s_l[(4 * kq + i) * kL + e] = acc[t][i] + p.cls_b[e];
+      if (e < E) s_l[(4 * kq + i) * kL + e] = acc[t][i] + cb[t];
   }
   __syncthreads();
   if (!live) return;
 
-  const float sc = scale_per_example ? scale_per_example[n] : scale;
   uint32_t key[MAXC];
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
@@ -318,23 +360,31 @@ __global__ __launch_bounds__(256) void hr_select_kernel(
 namespace {
 int64_t a256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
-// Whether the context rows, the classifier and the selection are launches of their own. Measured
-// over widths 64 to 1024, 64 to 512 experts and 1 to 2048 rows, both forms:
-//  - up to 64 rows (the small tiles of launch_router_logits) beyond width 128 or 256 experts:
-//    4 rows of width 256 15.6 against 18.2 us, 64 rows 19.9 against 22.0; at width 128 and 256
-//    experts they are equal, and the two launches win below;
-//  - up to 1024 rows where the width is a multiple of 512, which the classifier's 8 x 8 tiles
-//    need (width 512: 512 rows 27.4 against 30.8 us; width 384: 46.4 against 27.9).
-bool hr_split(int W, int E, int64_t rows) {
-  return (rows <= 64 && (W > 128 || E > 256)) || (rows <= 1024 && W % 512 == 0);
+// Whether the context rows, the classifier and the selection are launches of their own, from both
+// forms' times over widths 64 to 1024, 64 to 512 experts and 1 to 5120 rows:
+//  - never up to width 512 and 256 KB of classifier: a launch costs the host 3 us, which the
+//    classifier's reading alone by a CU does not reach (one example, width 512, 256 experts: 22.4
+//    against 27.9 us a call, 18.2 against 16.0 on the GPU);
+//  - beyond, up to 64 rows (the small tiles of launch_router_logits; width 768, 256 experts, 64 rows
+//    28.4 against 31.8 us a call, 160 rows 34.9 against 32), and up to 512 where the width is a
+//    multiple of 512, which the classifier's 8 x 8 tiles need (width 1024, 256 rows 29.1 against
+//    34.7, 1024 rows 50.0 against 45.9);
+//  - always where a bf16 array starts at an odd element: the context kernel loads single ones.
+bool hr_split(const moe_hr_predictor_params_v1& p, int64_t rows) {
+  const uintptr_t bases =
+      reinterpret_cast<uintptr_t>(p.ln_w) | reinterpret_cast<uintptr_t>(p.ln_b) |
+      reinterpret_cast<uintptr_t>(p.layer_emb) | reinterpret_cast<uintptr_t>(p.delta_emb);
+  if (bases & 3u) return true;
+  if (p.width <= 512 && p.width * p.num_experts <= 128 * 1024) return false;
+  return rows <= (p.width % 512 == 0 ? 512 : 64);
 }
 }  // namespace
 
 // Workspace sections: z [N][W + 1] fp32; in the split form also g [N * F][W] bf16 and logits
 // [N * F][E + 1] fp32.
-int64_t hr_predictor_workspace(int N, int W, int F, int E) {
-  const int64_t rows = (int64_t)N * F, z = a256((int64_t)N * (W + 1) * 4);
-  return hr_split(W, E, rows) ? z + a256(rows * W * 2) + a256(rows * (E + 1) * 4) : z;
+int64_t hr_predictor_workspace(int N, const moe_hr_predictor_params_v1& p) {
+  const int64_t rows = (int64_t)N * p.future_window, z = a256((int64_t)N * (p.width + 1) * 4);
+  return hr_split(p, rows) ? z + a256(rows * p.width * 2) + a256(rows * (p.num_experts + 1) * 4) : z;
 }
 
 hipError_t launch_hr_predictor(const uint16_t* x, int N, int H, const int32_t* layer_ids,
@@ -353,7 +403,7 @@ hipError_t launch_hr_predictor(const uint16_t* x, int N, int H, const int32_t* l
     err = hipGetLastError();
   }
   if (err != hipSuccess) return err;
-  if (hr_split(W, E, rows)) {
+  if (hr_split(p, rows)) {
     uint16_t* g = reinterpret_cast<uint16_t*>(ws + a256((int64_t)N * (W + 1) * 4));
     float* lg = reinterpret_cast<float*>(ws + a256((int64_t)N * (W + 1) * 4) +
                                          a256((int64_t)rows * W * 2));
@@ -376,9 +426,11 @@ hipError_t launch_hr_predictor(const uint16_t* x, int N, int H, const int32_t* l
                        rows, F, layer_ids, p, prior, scale, scale_per_example, top_k, out, ids);
     return hipGetLastError();
   };
-  if (p.num_experts <= 256)
-    return W <= 256 ? go(hr_rows_kernel<4, 4>) : go(hr_rows_kernel<16, 4>);
-  return W <= 256 ? go(hr_rows_kernel<4, 8>) : go(hr_rows_kernel<16, 8>);
+  if (E <= 256)
+    return W <= 256 ? go(hr_rows_kernel<4, 4>)
+                    : (W <= 512 ? go(hr_rows_kernel<8, 4>) : go(hr_rows_kernel<16, 4>));
+  return W <= 256 ? go(hr_rows_kernel<4, 8>)
+                  : (W <= 512 ? go(hr_rows_kernel<8, 8>) : go(hr_rows_kernel<16, 8>));
 }
 
 namespace {
@@ -417,7 +469,7 @@ extern "C" {
 
 int64_t moe_hr_predictor_workspace_bytes_v1(int32_t N, const moe_hr_predictor_params_v1* params) {
   if (!params || N < 0) return -1;
-  return hr_predictor_workspace(N, params->width, params->future_window, params->num_experts);
+  return hr_predictor_workspace(N, *params);
 }
 
 int moe_hr_predictor_v1(const uint16_t* hidden, int32_t N, const int32_t* layer_ids,
@@ -430,8 +482,7 @@ int moe_hr_predictor_v1(const uint16_t* hidden, int32_t N, const int32_t* layer_
   if (N == 0) return MOE_OK;
   if (!hidden || !layer_ids || !workspace || !topk_ids)
     return hr_fail(MOE_ERR_NULL, "NULL hidden, layer_ids, workspace or topk_ids");
-  if (workspace_bytes < hr_predictor_workspace(N, params->width, params->future_window,
-                                               params->num_experts))
+  if (workspace_bytes < hr_predictor_workspace(N, *params))
     return hr_fail(MOE_ERR_WORKSPACE, "workspace too small");
   if (!workspace_aligned(workspace)) return hr_fail(MOE_ERR_WORKSPACE, "workspace must be 256-byte aligned");
   const hipError_t e = launch_hr_predictor(hidden, N, params->hidden, layer_ids, *params, prior,

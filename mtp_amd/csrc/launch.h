@@ -196,7 +196,7 @@ constexpr int kPrefillBlockM = 128;
 constexpr int kAutoPrefillSlots = 2560;
 
 // HiddenResidualExpertPredictor forward (hr_predictor.hip).
-int64_t hr_predictor_workspace(int N, int W, int F, int E);
+int64_t hr_predictor_workspace(int N, const moe_hr_predictor_params_v1& p);
 hipError_t launch_hr_predictor(const uint16_t* x, int N, int H, const int32_t* layer_ids,
                                const moe_hr_predictor_params_v1& p, const float* prior, float scale,
                                const float* scale_per_example, int top_k, void* workspace,

@@ -434,8 +434,12 @@ def test_hidden_residual_predictor_matches_oracle(scope):
 @pytest.mark.parametrize("N,H,W,F,E,k", [(1, 64, 64, 1, 4, 2), (17, 520, 264, 3, 260, 16),
                                          (11, 2048, 72, 3, 40, 8), (6, 1024, 1024, 7, 512, 64),
                                          (40, 2056, 256, 1, 100, 1),
-                                         # the same in rows of the two-launch form
-                                         (31, 520, 264, 3, 260, 16), (150, 1024, 1024, 7, 512, 64)])
+                                         # every width and expert class of the two-launch form
+                                         (31, 520, 264, 3, 260, 16), (5, 512, 392, 3, 200, 8),
+                                         (9, 512, 136, 3, 400, 8), (200, 1024, 1024, 7, 256, 8),
+                                         (150, 1024, 1024, 7, 512, 64),
+                                         # four launches, a width of no multiple of 64
+                                         (5, 512, 776, 3, 40, 8)])
 def test_hidden_residual_predictor_tile_edges(N, H, W, F, E, k):
     from mtp_amd.predictor import HiddenResidualExpertPredictor
     _say(f"hidden-residual predictor N={N} H={H} W={W} F={F} E={E} k={k}")
@@ -454,9 +458,9 @@ def test_hidden_residual_predictor_tile_edges(N, H, W, F, E, k):
     _ids_match_up_to_near_ties(ids.cpu().numpy(), r_ids, r_out, 2e-2)
 
 
-# (N, W, F, E): the last row count of the four-launch form, by width and by experts; the last of
-# the widths whose classifier takes 8 x 8 tiles; the last example of the GEMV encoder
-@pytest.mark.parametrize("N,W,F,E", [(64, 256, 1, 256), (32, 128, 2, 300), (256, 512, 4, 64),
+# (N, W, F, E): the last row count of the four-launch form at a wide context, at a large classifier
+# and at a width whose classifier takes 8 x 8 tiles; the last example of the GEMV encoder
+@pytest.mark.parametrize("N,W,F,E", [(64, 768, 1, 64), (32, 384, 2, 400), (128, 512, 4, 512),
                                      (16, 64, 1, 64)])
 def test_hidden_residual_predictor_forms_agree(N, W, F, E):
     """An example's logits and experts are the same, up to the order of the fp32 sums, on both
@@ -475,10 +479,27 @@ def test_hidden_residual_predictor_forms_agree(N, W, F, E):
     _ids_match_up_to_near_ties(ids1[:N].cpu().numpy(), ids0.cpu().numpy(), out0.cpu().numpy(), 2e-2)
 
 
-@pytest.mark.parametrize("W,E", [(512, 256), (1024, 512)])
+def test_hidden_residual_predictor_parameters_at_odd_elements():
+    """bf16 parameters that start 2 bytes past a word give the aligned call's logits."""
+    from mtp_amd.predictor import HiddenResidualExpertPredictor
+    m = HiddenResidualExpertPredictor(hidden_size=512, num_experts=40, num_layers=5,
+                                      future_window=2, width=136, seed=4, device="cuda")
+    h = torch.randn(9, 512, device="cuda").to(torch.bfloat16)
+    lid = (torch.arange(9) % 5).to(torch.int32)
+    want = m(h, layer_ids=lid)
+    for name in ("ln_w", "ln_b", "layer_emb", "delta_emb"):
+        t = getattr(m, name)
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        flat[1:] = t.reshape(-1)
+        setattr(m, name, flat[1:].view(t.shape))
+        # the tolerance of the edges' test: an activation may round the other way
+        assert (m(h, layer_ids=lid) - want).abs().max() <= 1e-2, name
+
+
+@pytest.mark.parametrize("W,E", [(768, 256), (1024, 512)])
 def test_one_example_is_not_priced_as_many(W, E):
     """One row of a wide classifier is spread over the chip: a call costs under half of 512 examples
-    (2048 rows), which read the same weights (measured 0.40 and 0.25 of them; 0.63 and 0.60 where
+    (2048 rows), which read the same weights (measured 0.35 and 0.25 of them; 0.57 and 0.60 where
     one workgroup reads the whole classifier)."""
     from mtp_amd.predictor import HiddenResidualExpertPredictor
     from tests.helpers import graph_us
