@@ -91,30 +91,49 @@ __global__ __launch_bounds__(64 * kEncWaves) void hr_encoder_kernel(
   }
 }
 
+// NW consecutive dwords at byte offset `off`, one load.
+template <int NW>
+MOE_DEV void ld_words(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t (&o)[NW]) {
+  static_assert(NW == 1 || NW == 2 || NW == 4, "one buffer load");
+  if constexpr (NW == 4) {
+    const u32x4 v = buf_ld128(r, off);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = v[j];
+  } else if constexpr (NW == 2) {
+    const u32x2 v = buf_ld64(r, off);
+    o[0] = v[0];
+    o[1] = v[1];
+  } else {
+    o[0] = buf_ld32(r, off);
+  }
+}
+
 // 16 context rows r = n * F + d per workgroup, one wave per row: SiLU, LayerNorm (fp32
 // statistics), embeddings and SiLU of the row into LDS as bf16; the 16 x E classifier tile on MFMA
 // (wave w the expert tiles w, w + 16); then v = (prior ? prior[r] : 0) + scale_n * logits[r],
 // optionally written to out, and the top-k of v by (value, lower id), again one wave per row, so
 // that the 16 selections of a workgroup run side by side (each is a serial chain of top_k rounds).
 // What bounds it is the memory round trips of that chain, so every operand of the context row, the
-// prior, the bias and the first classifier steps are loaded together, four columns a lane (one
+// prior, the bias and the first classifier steps are loaded together, four columns a lane, two up to
+// width 128 (one
 // column a lane with the loads behind their range checks: one example 12.4 us against 10.6 at
 // width 256, 20.3 against 14.2 at width 512), and a wave keeps kRing classifier steps in flight.
 // NC, MAXC: 64-lane columns of the width and of the experts. The F rows of one example repeat its
 // LayerNorm: cheaper than another launch. 64 VGPRs where that fits: two workgroups per CU (5120
-// rows of width 128: 33.5 us, with one 36.7).
+// rows of width 64 at four columns a lane 29.5 us, with one workgroup 32.0).
 constexpr int kRows = 16;
 template <int NC, int MAXC>
-__global__ __launch_bounds__(64 * kRows, NC + MAXC == 8 ? 8 : 4) void hr_rows_kernel(
+__global__ __launch_bounds__(64 * kRows, NC + MAXC <= 8 ? 8 : 4) void hr_rows_kernel(
     const float* __restrict__ z, int rows, int F, const int32_t* __restrict__ layer_ids,
     moe_hr_predictor_params_v1 p, const float* __restrict__ prior, float scale,
     const float* __restrict__ scale_per_example, int top_k, float* __restrict__ out,
     int32_t* __restrict__ ids) {
   constexpr int kG = 64 * NC + 8, kL = 64 * MAXC + 4;  // row strides (16-byte rows, odd quads)
   constexpr int TPW = MAXC / 4;                        // expert tiles per wave
-  constexpr int NQ = NC / 4;                           // column quads per lane
+  constexpr int CPL = NC < 4 ? NC : 4, NQ = NC / CPL;  // columns of a load, loads per lane
   // classifier k-steps of 32: in all, in the ring of a wave, and of these loaded before the context
-  constexpr int kSteps = 2 * NC, kRing = 16 / TPW < kSteps ? 16 / TPW : kSteps, kFirst = 8 / TPW;
+  constexpr int kSteps = 2 * NC, kRing = 16 / TPW < kSteps ? 16 / TPW : kSteps,
+                kFirst = 8 / TPW < kRing ? 8 / TPW : kRing;
   __shared__ __attribute__((aligned(16))) uint16_t s_g[kRows * kG];
   __shared__ float s_l[kRows * kL];
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
@@ -127,7 +146,7 @@ __global__ __launch_bounds__(64 * kRows, NC + MAXC == 8 ? 8 : 4) void hr_rows_ke
   const bool layer_ok = layer >= 0 && layer < p.num_layers;  // else the embedding reads zeros
   const float sc = scale_per_example ? scale_per_example[n] : scale;
 
-  // The context row's operands (lane: columns 4 (lane + 64 i) ..; past the width zeros, without a
+  // The context row's operands (lane: columns CPL (lane + 64 i) ..; past the width zeros, without a
   // memory access), the prior, the classifier's bias and its first chunk: one memory latency.
   const uint32_t wb = (uint32_t)W * 2u;
   const __amdgpu_buffer_rsrc_t zr = buf_rsrc(z + (int64_t)n * (W + 1), 2u * wb);
@@ -136,17 +155,17 @@ __global__ __launch_bounds__(64 * kRows, NC + MAXC == 8 ? 8 : 4) void hr_rows_ke
   const __amdgpu_buffer_rsrc_t ler =
       buf_rsrc(p.layer_emb + (int64_t)(layer_ok ? layer : 0) * W, layer_ok ? wb : 0u);
   const __amdgpu_buffer_rsrc_t der = buf_rsrc(p.delta_emb + (int64_t)d * W, wb);
-  u32x4 zq[NQ], bq[NQ];
-  u32x2 lw[NQ], lb[NQ], le[NQ], de[NQ];
+  uint32_t zq[NQ][CPL], bq[NQ][CPL], lw[NQ][CPL / 2], lb[NQ][CPL / 2], le[NQ][CPL / 2],
+      de[NQ][CPL / 2];
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
-    const uint32_t q = (uint32_t)(lane + 64 * i);
-    zq[i] = buf_ld128(zr, q * 16u);
-    bq[i] = buf_ld128(br, q * 16u);
-    lw[i] = buf_ld64(lwr, q * 8u);
-    lb[i] = buf_ld64(lbr, q * 8u);
-    le[i] = buf_ld64(ler, q * 8u);
-    de[i] = buf_ld64(der, q * 8u);
+    const uint32_t o = (uint32_t)(CPL * 2 * (lane + 64 * i));
+    ld_words(zr, 2u * o, zq[i]);
+    ld_words(br, 2u * o, bq[i]);
+    ld_words(lwr, o, lw[i]);
+    ld_words(lbr, o, lb[i]);
+    ld_words(ler, o, le[i]);
+    ld_words(der, o, de[i]);
   }
   const __amdgpu_buffer_rsrc_t pr = buf_rsrc(prior ? prior + (int64_t)(live ? row : 0) * E : nullptr,
                                              prior && live ? (uint32_t)E * 4u : 0u);
@@ -174,41 +193,48 @@ __global__ __launch_bounds__(64 * kRows, NC + MAXC == 8 ? 8 : 4) void hr_rows_ke
   for (int i = 0; i < kFirst; ++i) load_cls(i);
   __builtin_amdgcn_sched_barrier(0);
 
-  float a[4 * NQ], sum = 0.0f;
+  float a[NQ][CPL], sum = 0.0f;
 #pragma unroll
   for (int i = 0; i < NQ; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < CPL; ++j) {
       const float zb = bf16_round(__uint_as_float(zq[i][j]) + __uint_as_float(bq[i][j]));
-      // a column past the width has z = bias = 0 and silu(0) = 0
-      a[4 * i + j] = bf16_round(zb / (1.0f + expf(-zb)));
-      sum += a[4 * i + j];
+      a[i][j] = bf16_round(zb / (1.0f + expf(-zb)));  // past the width silu(0) = 0
+      sum += a[i][j];
     }
   const float mean = bfly_sum(sum) / (float)W;
   float sq = 0.0f;
 #pragma unroll
   for (int i = 0; i < NQ; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float dv = 4 * (lane + 64 * i) < W ? a[4 * i + j] - mean : 0.0f;
+    for (int j = 0; j < CPL; ++j) {
+      const float dv = CPL * (lane + 64 * i) < W ? a[i][j] - mean : 0.0f;
       sq = __builtin_fmaf(dv, dv, sq);
     }
   const float var = bfly_sum(sq) / (float)W;
   const float rstd = 1.0f / sqrtf(var + p.ln_eps);
-  auto el = [](u32x2 v, int j) { return (j & 1) ? bf16hi_to_f32(v[j >> 1]) : bf16lo_to_f32(v[j >> 1]); };
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
-    const uint32_t in = 0u - (uint32_t)(4 * (lane + 64 * i) < W);
-    uint32_t g[4];
+    const uint32_t in = 0u - (uint32_t)(CPL * (lane + 64 * i) < W);
+    uint32_t g[CPL / 2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float s = bf16_round((a[4 * i + j] - mean) * rstd * el(lw[i], j) + el(lb[i], j));
-      const float sl = bf16_round(s + el(le[i], j));
-      const float c = bf16_round(sl + el(de[i], j));
-      g[j] = f32_to_bf16_rne(c / (1.0f + expf(-c))) & in;
+    for (int w = 0; w < CPL / 2; ++w) {
+      uint32_t half[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        auto el = [&](uint32_t v) { return h ? bf16hi_to_f32(v) : bf16lo_to_f32(v); };
+        const float s = bf16_round((a[i][2 * w + h] - mean) * rstd * el(lw[i][w]) + el(lb[i][w]));
+        const float sl = bf16_round(s + el(le[i][w]));
+        const float c = bf16_round(sl + el(de[i][w]));
+        half[h] = f32_to_bf16_rne(c / (1.0f + expf(-c)));
+      }
+      g[w] = (half[0] | (half[1] << 16)) & in;
     }
-    *reinterpret_cast<u32x2*>(s_g + wv * kG + 4 * (lane + 64 * i)) =
-        u32x2{g[0] | (g[1] << 16), g[2] | (g[3] << 16)};
+    uint16_t* dst = s_g + wv * kG + CPL * (lane + 64 * i);
+    if constexpr (CPL == 4)
+      *reinterpret_cast<u32x2*>(dst) = u32x2{g[0], g[1]};
+    else
+      *reinterpret_cast<uint32_t*>(dst) = g[0];
   }
 #pragma unroll
   for (int i = kFirst; i < kRing; ++i) load_cls(i);
@@ -426,11 +452,14 @@ hipError_t launch_hr_predictor(const uint16_t* x, int N, int H, const int32_t* l
                        rows, F, layer_ids, p, prior, scale, scale_per_example, top_k, out, ids);
     return hipGetLastError();
   };
-  if (E <= 256)
-    return W <= 256 ? go(hr_rows_kernel<4, 4>)
-                    : (W <= 512 ? go(hr_rows_kernel<8, 4>) : go(hr_rows_kernel<16, 4>));
-  return W <= 256 ? go(hr_rows_kernel<4, 8>)
-                  : (W <= 512 ? go(hr_rows_kernel<8, 8>) : go(hr_rows_kernel<16, 8>));
+  if (E <= 256) {
+    if (W <= 128) return go(hr_rows_kernel<2, 4>);
+    if (W <= 256) return go(hr_rows_kernel<4, 4>);
+    return W <= 512 ? go(hr_rows_kernel<8, 4>) : go(hr_rows_kernel<16, 4>);
+  }
+  if (W <= 128) return go(hr_rows_kernel<2, 8>);
+  if (W <= 256) return go(hr_rows_kernel<4, 8>);
+  return W <= 512 ? go(hr_rows_kernel<8, 8>) : go(hr_rows_kernel<16, 8>);
 }
 
 namespace {

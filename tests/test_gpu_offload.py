@@ -436,7 +436,8 @@ def test_hidden_residual_predictor_matches_oracle(scope):
                                          (40, 2056, 256, 1, 100, 1),
                                          # every width and expert class of the two-launch form
                                          (31, 520, 264, 3, 260, 16), (5, 512, 392, 3, 200, 8),
-                                         (9, 512, 136, 3, 400, 8), (200, 1024, 1024, 7, 256, 8),
+                                         (9, 512, 136, 3, 400, 8), (30, 512, 104, 2, 300, 8),
+                                         (200, 1024, 1024, 7, 256, 8),
                                          (150, 1024, 1024, 7, 512, 64),
                                          # four launches, a width of no multiple of 64
                                          (5, 512, 776, 3, 40, 8)])
