@@ -195,12 +195,13 @@ __global__ __launch_bounds__(256) void dequant_kernel(ProjDev p, const int32_t* 
   }
 }
 
-// Whether the tile kernel is the faster one, from both kernels' times over 2^14 to 2^22 packed words
-// of 8 to 2048 k and 8 to 2048 columns (in ps beyond a launch of 3.4 us). The one-thread-per-word
-// kernel takes 10 per word (7 in long rows of words) and 3 per thread, and 256 threads cover a
-// row's columns. The tile kernel takes a fixed chain of loads, LDS and stores, plus a share per tile
-// of 32 packed rows x 64 columns, full or not, and with g_idx of the tile's table. bf16 linear: 1 expert of 512 x 512 3.7 against 6.1 us, 2 of 2048 x 512
-// 8.0 against 6.8, 4 of them 11.1 against 7.4, 256 of 24 x 512 8.7 against 16.0.
+// Whether the tile kernel is the faster one, from both kernels' times over 2^14 to 2^22 packed
+// words of 8 to 2048 k and 8 to 2048 columns (in ps beyond a launch of 3.4 us). The
+// one-thread-per-word kernel takes 10 per word (7 in long rows of words) and 3 per thread, and 256
+// threads cover a row's columns. The tile kernel takes a fixed chain of loads, LDS and stores, plus
+// a share per tile of 32 packed rows x 64 columns, full or not, and with g_idx of the tile's table.
+// bf16 linear: 1 expert of 512 x 512 3.7 against 6.1 us, 2 of 2048 x 512 8.0 against 6.8, 4 of them
+// 11.1 against 7.4, 256 of 24 x 512 8.7 against 16.0.
 bool tile_pays(int64_t E, int64_t K, int64_t N, int64_t G, bool linear, bool fp32, bool idx) {
   const int64_t words = E * (K / 8) * N, threads = E * (K / 8) * ((N + 255) / 256 * 256);
   const int64_t tiles = E * ((K / 8 + kTileR - 1) / kTileR) * ((N + kTileC - 1) / kTileC);
